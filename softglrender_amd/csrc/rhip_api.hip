@@ -19,20 +19,13 @@
 
 #include "rhip.h"
 #include "rhip_host.h"
+#include "rhip_launch.h"
 #include "rhip_neural.h"
 #include "rhip_lines.h"
 
 #include <hipcub/hipcub.hpp>
 
 using namespace rhip;
-
-/* Every kernel launch goes through this macro (one place to change how kernels are started). */
-/* a comma inside a macro argument (template argument lists) */
-#define RHIP_COMMA ,
-
-#ifndef RHIP_LAUNCH
-#define RHIP_LAUNCH(kern, grid, block, stream, ...) kern<<<(grid), (block), 0, (stream)>>>(__VA_ARGS__)
-#endif
 
 namespace rhip {
 
@@ -222,95 +215,6 @@ struct Timer {
   }
 };
 
-/* Wavefronts per tile of a single draw's two-phase raster: four for 4x targets,
- * two without MSAA, whose tiles carry a quarter of the samples (measured on the
- * C2 frame: 2048^2 shadow pass 126 -> 111 us with two; the 4x pass 114 -> 152 us). */
-template <int S>
-constexpr int visWaves() {
-  return S == 4 ? 4 : 2;
-}
-
-/* Two-phase raster: coarse hierarchical Z, then visibility and depth per tile. */
-template <int S>
-void launchVis(rhip_device d, const DrawParams &P, int ntiles, int ncoarse, hipStream_t st) {
-  const int f = P.st.depthFunc;
-  {
-    Timer tm(d, "k_hiz_coarse");
-    if (f == 4 || f == 6) {
-      RHIP_LAUNCH(k_hiz_coarse<S RHIP_COMMA true>, ncoarse, 256, st, P);
-    } else {
-      RHIP_LAUNCH(k_hiz_coarse<S RHIP_COMMA false>, ncoarse, 256, st, P);
-    }
-  }
-  Timer tm(d, S == 4 ? "k_raster_vis_msaa4" : "k_raster_vis");
-  switch (f) {
-    case 1: RHIP_LAUNCH(k_raster_vis<S RHIP_COMMA VIS_LESS RHIP_COMMA kTile RHIP_COMMA visWaves<S>()>, ntiles, 64 * visWaves<S>(), st, P); break;
-    case 3: RHIP_LAUNCH(k_raster_vis<S RHIP_COMMA VIS_LEQUAL RHIP_COMMA kTile RHIP_COMMA visWaves<S>()>, ntiles, 64 * visWaves<S>(), st, P); break;
-    case 4: RHIP_LAUNCH(k_raster_vis<S RHIP_COMMA VIS_GREATER RHIP_COMMA kTile RHIP_COMMA visWaves<S>()>, ntiles, 64 * visWaves<S>(), st, P); break;
-    default: RHIP_LAUNCH(k_raster_vis<S RHIP_COMMA VIS_GEQUAL RHIP_COMMA kTile RHIP_COMMA visWaves<S>()>, ntiles, 64 * visWaves<S>(), st, P); break;
-  }
-}
-
-/* Shading of the fragments the two-phase raster queued. */
-template <int S>
-void launchShade(const DrawParams &P, int grid, int need_deriv, hipStream_t st) {
-  switch (P.shading) {
-    case RHS_SHADING_BASIC: RHIP_LAUNCH(k_shade<S RHIP_COMMA RHS_SHADING_BASIC>, grid, 256, st, P, need_deriv); break;
-    case RHS_SHADING_BLINN_PHONG:
-      RHIP_LAUNCH(k_shade<S RHIP_COMMA RHS_SHADING_BLINN_PHONG>, grid, 256, st, P, need_deriv);
-      break;
-    case RHS_SHADING_BLINN_PHONG_DIR:
-      RHIP_LAUNCH(k_shade<S RHIP_COMMA RHS_SHADING_BLINN_PHONG_DIR>, grid, 256, st, P, need_deriv);
-      break;
-    case RHS_SHADING_PBR: RHIP_LAUNCH(k_shade<S RHIP_COMMA RHS_SHADING_PBR>, grid, 256, st, P, need_deriv); break;
-    default: RHIP_LAUNCH(k_shade<S RHIP_COMMA RHS_SHADING_VERTEX_COLOR>, grid, 256, st, P, need_deriv); break;
-  }
-}
-
-/* Shading of the listed ordered raster's fragments, and its fallback for tiles that did not fit. */
-template <int S>
-void launchOrdShade(const DrawParams &P, int grid, int need_deriv, hipStream_t st) {
-  switch (P.shading) {
-    case RHS_SHADING_BASIC: RHIP_LAUNCH(k_ord_shade<S RHIP_COMMA RHS_SHADING_BASIC>, grid, 256, st, P, need_deriv); break;
-    case RHS_SHADING_BLINN_PHONG:
-      RHIP_LAUNCH(k_ord_shade<S RHIP_COMMA RHS_SHADING_BLINN_PHONG>, grid, 256, st, P, need_deriv);
-      break;
-    case RHS_SHADING_BLINN_PHONG_DIR:
-      RHIP_LAUNCH(k_ord_shade<S RHIP_COMMA RHS_SHADING_BLINN_PHONG_DIR>, grid, 256, st, P, need_deriv);
-      break;
-    case RHS_SHADING_PBR: RHIP_LAUNCH(k_ord_shade<S RHIP_COMMA RHS_SHADING_PBR>, grid, 256, st, P, need_deriv); break;
-    case RHS_SHADING_IBL_IRRADIANCE:
-    case RHS_SHADING_IBL_PREFILTER:
-      /* one wavefront per fragment: `grid` blocks of 256 lanes cover the fragments one lane each */
-      RHIP_LAUNCH(k_ord_shade_ibl<S>, std::min(grid * 64, 16384), 256, st, P, need_deriv);
-      break;
-    case RHS_SHADING_SKYBOX:
-    case RHS_SHADING_FXAA: RHIP_LAUNCH(k_ord_shade<S RHIP_COMMA kShadingEnv>, grid, 256, st, P, need_deriv); break;
-    default: RHIP_LAUNCH(k_ord_shade<S RHIP_COMMA RHS_SHADING_VERTEX_COLOR>, grid, 256, st, P, need_deriv); break;
-  }
-}
-
-template <int S>
-void launchOrdRest(const DrawParams &P, int grid, int need_deriv, hipStream_t st) {
-  switch (P.shading) {
-    case RHS_SHADING_BASIC: RHIP_LAUNCH(k_ord_rest<S RHIP_COMMA RHS_SHADING_BASIC>, grid, 256, st, P, need_deriv); break;
-    case RHS_SHADING_BLINN_PHONG:
-      RHIP_LAUNCH(k_ord_rest<S RHIP_COMMA RHS_SHADING_BLINN_PHONG>, grid, 256, st, P, need_deriv);
-      break;
-    case RHS_SHADING_BLINN_PHONG_DIR:
-      RHIP_LAUNCH(k_ord_rest<S RHIP_COMMA RHS_SHADING_BLINN_PHONG_DIR>, grid, 256, st, P, need_deriv);
-      break;
-    case RHS_SHADING_PBR: RHIP_LAUNCH(k_ord_rest<S RHIP_COMMA RHS_SHADING_PBR>, grid, 256, st, P, need_deriv); break;
-    case RHS_SHADING_SKYBOX:
-    case RHS_SHADING_IBL_IRRADIANCE:
-    case RHS_SHADING_IBL_PREFILTER:
-    case RHS_SHADING_FXAA: RHIP_LAUNCH(k_ord_rest<S RHIP_COMMA kShadingEnv>, grid, 256, st, P, need_deriv); break;
-    default: RHIP_LAUNCH(k_ord_rest<S RHIP_COMMA RHS_SHADING_VERTEX_COLOR>, grid, 256, st, P, need_deriv); break;
-  }
-}
-
-/* Listed ordered raster of a draw that writes no depth. */
-
 /* The multisample resolve a draw ends with (RendererSoft.cpp:161-163): launched now, or, for rhip_draw,
  * left pending until something may read the resolved image (checkDev, drawOne). */
 }  // namespace
@@ -340,6 +244,7 @@ static void resolveAfterDraw(rhip_device d, const DrawParams &P, unsigned grid, 
   RHIP_LAUNCH(k_resolve, grid, 256, s, P);
 }
 
+/* Listed ordered raster of a draw that writes no depth. */
 template <int S>
 void launchListed(rhip_device d, const DrawParams &P, int need_deriv, hipStream_t st) {
   const size_t npx = (size_t)P.fb_w * P.fb_h;
@@ -360,43 +265,6 @@ void launchListed(rhip_device d, const DrawParams &P, int need_deriv, hipStream_
     launchOrdRest<S>(P, std::min(P.ntiles, 512), need_deriv, st);
   }
   if (S == 4 && P.color) resolveAfterDraw(d, P, (unsigned)std::min<size_t>(blocks(npx, 256), 4096), st);
-}
-
-/* Ordered raster (every state the two-phase raster does not take). */
-template <int S>
-void launchOrdered(const DrawParams &P, int ntiles, int need_deriv, int flush_each, hipStream_t st) {
-  switch (P.shading) {
-    case RHS_SHADING_BASIC: {
-#define K_ORD k_raster_ord<S, RHS_SHADING_BASIC>
-      RHIP_LAUNCH(K_ORD, ntiles, 256, st, P, need_deriv, flush_each);
-#undef K_ORD
-      break;
-    }
-    case RHS_SHADING_BLINN_PHONG: {
-#define K_ORD k_raster_ord<S, RHS_SHADING_BLINN_PHONG>
-      RHIP_LAUNCH(K_ORD, ntiles, 256, st, P, need_deriv, flush_each);
-#undef K_ORD
-      break;
-    }
-    case RHS_SHADING_BLINN_PHONG_DIR: {
-#define K_ORD k_raster_ord<S, RHS_SHADING_BLINN_PHONG_DIR>
-      RHIP_LAUNCH(K_ORD, ntiles, 256, st, P, need_deriv, flush_each);
-#undef K_ORD
-      break;
-    }
-    case RHS_SHADING_PBR: {
-#define K_ORD k_raster_ord<S, RHS_SHADING_PBR>
-      RHIP_LAUNCH(K_ORD, ntiles, 256, st, P, need_deriv, flush_each);
-#undef K_ORD
-      break;
-    }
-    default: {
-#define K_ORD k_raster_ord<S, RHS_SHADING_VERTEX_COLOR>
-      RHIP_LAUNCH(K_ORD, ntiles, 256, st, P, need_deriv, flush_each);
-#undef K_ORD
-      break;
-    }
-  }
 }
 
 }  // namespace
@@ -1166,10 +1034,14 @@ int drawOne(rhip_device d, const rhip_draw_desc *dd, bool no_alloc) {
   if (sh.two_phase) {
     const int ncoarse = P.coarse_x * P.coarse_y;
     const size_t njobs = (size_t)fbw * fbh * samples;
-    if (samples == 4)
-      launchVis<4>(d, P, ntiles, ncoarse, s);
-    else
-      launchVis<1>(d, P, ntiles, ncoarse, s);
+    {
+      Timer tm(d, "k_hiz_coarse");
+      samples == 4 ? launchHiz<4>(P, ncoarse, s) : launchHiz<1>(P, ncoarse, s);
+    }
+    {
+      Timer tm(d, samples == 4 ? "k_raster_vis_msaa4" : "k_raster_vis");
+      samples == 4 ? launchVis<4>(P, ntiles, s) : launchVis<1>(P, ntiles, s);
+    }
     if (P.color) {
       const int grid = (int)std::min<size_t>(blocks(njobs, 256), 4096);
       if (P.shading == RHS_SHADING_NEURAL_PBR) {
