@@ -896,14 +896,11 @@ __device__ __forceinline__ IrrSetup irrSetup(const Frag &f) {
   s.up = nrm3b(cross3(s.N, s.right));
   return s;
 }
-/* Term k of the sum (phi index k / ntheta, theta index k % ntheta): the sample's
+/* A term of the sum from the sines and cosines of its loop angles: the sample's
  * colour times cos(theta), and sin(theta). The reference build fuses the last
  * product into the running sum (irrAdd), and the sample vector into two
  * multiply-adds. */
-__device__ __forceinline__ float4 irrTerm(const DrawParams &P, const IrrSetup &s, int k) {
-  const IblTables &T = *P.ibl;
-  const int i = k / T.ntheta, j = k - i * T.ntheta;
-  const float sp = T.sphi[i], cp = T.cphi[i], st = T.stheta[j], ct = T.ctheta[j];
+__device__ __forceinline__ float4 irrTerm(const DrawParams &P, const IrrSetup &s, float sp, float cp, float st, float ct) {
   const f3 ts{st * cp, st * sp, ct};
   const f3 sv{fmaf(s.N.x, ts.z, fmaf(s.up.x, ts.y, s.right.x * ts.x)),
               fmaf(s.N.y, ts.z, fmaf(s.up.y, ts.y, s.right.y * ts.x)),
@@ -920,13 +917,14 @@ __device__ __forceinline__ RGBAf irrFinish(f3 irr, float nr) {
 }
 __device__ RGBAf fsIrradiance(const DrawParams &P, const Frag &f) {
   const IrrSetup s = irrSetup(f);
-  const int n = P.ibl->nphi * P.ibl->ntheta;
+  const IblTables &T = *P.ibl;
   f3 irr{0.f, 0.f, 0.f};
   float nr = 0.f;
-  for (int k = 0; k < n; k++) {
-    irr = irrAdd(irr, irrTerm(P, s, k));
-    nr += 1.f;
-  }
+  for (int i = 0; i < T.nphi; i++)
+    for (int j = 0; j < T.ntheta; j++) {
+      irr = irrAdd(irr, irrTerm(P, s, T.sphi[i], T.cphi[i], T.stheta[j], T.ctheta[j]));
+      nr += 1.f;
+    }
   return irrFinish(irr, nr);
 }
 
@@ -954,15 +952,19 @@ __device__ __forceinline__ PrefSetup prefSetup(const DrawParams &P, const Frag &
   s.saTexel = 4.0f * kPI / (6.0f * res * res);
   return s;
 }
-/* Sample i: the source texel's colour and N.L (the sample counts only when N.L > 0). */
-__device__ __forceinline__ float4 prefSample(const DrawParams &P, const PrefSetup &s, uint32_t i) {
+/* Sample i's half vector in tangent space: it depends on the draw's roughness only. */
+__device__ __forceinline__ f3 prefHalf(const DrawParams &P, uint32_t i) {
   const IblTables &T = *P.ibl;
-  const f3 N = s.N, V = s.V, tangent = s.tangent, bitangent = s.bitangent;
-  const float ra2 = s.ra2;
+  const float a = P.u.aux[1] * P.u.aux[1], ra2 = a * a;
   const float xiy = (float)((double)__builtin_bitreverse32(i) * 2.3283064365386963e-10);
   const float cosT = sqrtf((1.0f - xiy) / fmaf(ra2 - 1.0f, xiy, 1.0f));
   const float sinT = sqrtf(fmaf(-cosT, cosT, 1.0f));
-  const f3 Ht{T.hcos[i] * sinT, T.hsin[i] * sinT, cosT};
+  return {T.hcos[i] * sinT, T.hsin[i] * sinT, cosT};
+}
+/* The sample of half vector Ht: the source texel's colour and N.L (the sample counts only when N.L > 0). */
+__device__ __forceinline__ float4 prefSample(const DrawParams &P, const PrefSetup &s, f3 Ht) {
+  const f3 N = s.N, V = s.V, tangent = s.tangent, bitangent = s.bitangent;
+  const float ra2 = s.ra2;
   const f3 H = nrm3b({fmaf(N.x, Ht.z, fmaf(bitangent.x, Ht.y, tangent.x * Ht.x)),
                       fmaf(N.y, Ht.z, fmaf(bitangent.y, Ht.y, tangent.y * Ht.x)),
                       fmaf(N.z, Ht.z, fmaf(bitangent.z, Ht.y, tangent.z * Ht.x))});
@@ -984,7 +986,7 @@ __device__ RGBAf fsPrefilter(const DrawParams &P, const Frag &f) {
   f3 acc{0.f, 0.f, 0.f};
   float tw = 0.f;
   for (uint32_t i = 0; i < 1024u; i++) {
-    const float4 t = prefSample(P, s, i);
+    const float4 t = prefSample(P, s, prefHalf(P, i));
     if (t.w > 0.0f) {
       acc = {fmaf(t.x, t.w, acc.x), fmaf(t.y, t.w, acc.y), fmaf(t.z, t.w, acc.z)};
       tw += t.w;
