@@ -1,0 +1,91 @@
+"""Texture sampling and the IBL precompute at the sizes where their kernels change path, identical to the checker."""
+import math
+import struct
+
+import numpy as np
+import pytest
+
+import oracle
+from softglrender_amd import scenes
+from softglrender_amd import stream as S
+from softglrender_amd.replay import replay
+
+from .util import assert_identical
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(renderer, sc, layouts=None):
+    got, _ = replay(renderer, sc.stream.bytes(), layouts=layouts)
+    out, _ = oracle.cpu_ref_replay(sc.stream.bytes(), sc.stream.output_bytes(), exact_math=False)
+    assert_identical(got, sc.stream.split_outputs(out), sc.name)
+
+
+def _textured(wrap, filt, tw, th, seed):
+    """A sphere with a tw x th texture whose coordinates run from -2 to 3, near enough that some of it is magnified
+    (LOD 0) and some minified."""
+    rng = np.random.default_rng(seed)
+    st = S.Stream()
+    v, idx = scenes.uv_sphere(24, 12)
+    v[:, 4:6] = v[:, 4:6] * 5.0 - 2.0
+    st.texture(1, tw, th, mipmaps=filt > S.FILTER_LINEAR, filter_min=filt, filter_mag=S.FILTER_LINEAR, wrap=wrap,
+               border=S.BORDER_WHITE, usage=S.USAGE_SAMPLER | S.USAGE_UPLOAD)
+    st.tex_data(1, [rng.integers(0, 256, (th, tw, 4), dtype=np.uint8)])
+    st.vao(1, v, idx)
+    st.texture(2, 150, 110, usage=S.USAGE_COLOR)
+    st.tex_init(2)
+    st.texture(3, 150, 110, format=S.FMT_FLOAT32, usage=S.USAGE_DEPTH)
+    st.tex_init(3)
+    st.fbo(1, color=2, depth=3)
+    st.frame()
+    eye = (0.3, 0.2, 1.7)
+    mvp = scenes.projection(math.radians(60.0), 150 / 110, 0.1) @ scenes.look_at(eye, (0, 0, 0), (0, 1, 0))
+    st.begin(1, True, True, (0, 0, 0, 0), 1.0)
+    st.viewport(0, 0, 150, 110)
+    st.draw(1, S.SHADING_BLINN_PHONG_DIR, S.DEF_ALBEDO, scenes._common_states(S.DEPTH_LESS),
+            S.uniforms_model(np.eye(4), mvp), S.uniforms_scene((0.6, 0.6, 0.6), eye, (1, 1, 1), (0.5, 0.5, 0.5)),
+            S.uniforms_material(1, 0, 0, 1.0, 0.2, (1, 1, 1, 1)), samplers=[(S.SLOT_ALBEDO, 1)])
+    st.end()
+    st.read(2)
+    return scenes.Scene("textured", st, 150, 110, False)
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("wrap", [S.WRAP_REPEAT, S.WRAP_MIRRORED_REPEAT, S.WRAP_CLAMP_TO_EDGE, S.WRAP_CLAMP_TO_BORDER])
+def test_footprint_matches_checker(renderer, wrap, layout):
+    """Every wrap mode and layout on powers of two, odd sizes and a single texel, bilinear and trilinear."""
+    for k, (tw, th) in enumerate(((64, 32), (37, 51), (1, 1))):
+        for filt in (S.FILTER_LINEAR, S.FILTER_LINEAR_MIPMAP_LINEAR):
+            print(f"[gpu] wrap {wrap} layout {layout} {tw}x{th} filter {filt}", flush=True)
+            _check(renderer, _textured(wrap, filt, tw, th, 7 + k), {1: layout})
+
+
+@pytest.mark.parametrize("size", [46, 67, 129])
+def test_ibl_groups_match_checker(renderer, size):
+    """One prefiltered face of a size whose fragments are taken 2, 4 or 16 to a workgroup (the last group not full),
+    and one irradiance face (1 to a workgroup)."""
+    print(f"[gpu] prefilter face of {size}^2", flush=True)
+    st = S.Stream()
+    v, idx = scenes.cube_mesh()
+    st.vao(1, v, idx)
+    st.texture(10, 16, 16, type=S.TEX_CUBE, mipmaps=True, usage=S.USAGE_SAMPLER | S.USAGE_UPLOAD,
+               filter_min=S.FILTER_LINEAR_MIPMAP_LINEAR, filter_mag=S.FILTER_LINEAR, wrap=S.WRAP_CLAMP_TO_EDGE)
+    st.tex_data(10, scenes.env_cube_faces(16, 3))
+    st.frame()
+    proj = scenes.projection(math.radians(90.0), 1.0, 0.1)
+    jobs = ((11, size, S.SHADING_IBL_PREFILTER, struct.pack("<2f", 16.0, 0.4) + bytes(40)),
+            (12, 5, S.SHADING_IBL_IRRADIANCE, bytes(48)))
+    for face, (tex, n, shading, mat) in enumerate(jobs):
+        center, up = scenes._CUBE_VIEWS[face]
+        turn = np.eye(4)
+        turn[:3, :3] = scenes.look_at((0, 0, 0), center, up)[:3, :3]
+        st.texture(tex, n, n, usage=S.USAGE_COLOR)
+        st.tex_init(tex)
+        st.fbo(tex, color=tex)
+        st.begin(tex, True, False, (0, 0, 0, 0), 1.0)
+        st.viewport(0, 0, n, n)
+        st.draw(1, shading, 0, S.RenderStates(), S.uniforms_model(np.eye(4), proj @ turn), bytes(64), mat,
+                samplers=[(S.SLOT_CUBE, 10)])
+        st.end()
+        st.read(tex)
+    _check(renderer, scenes.Scene(f"ibl face {size}", st, size, size, False))
