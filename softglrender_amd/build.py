@@ -22,8 +22,8 @@ HIP_FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffp-contr
              "-I", os.path.join(ROOT, "include"), "-I", CSRC]
 
 TARGETS = {
-    "librhip.so": ["rhip_api.hip", "rhip_raster.hip", "rhip_shade.hip", "rhip_ord1.hip", "rhip_ord4.hip", "rhip_batch.hip",
-                   "rhip_batch_vis1.hip", "rhip_batch_vis4.hip", "rhip_libm.hip"],
+    "librhip.so": ["rhip_api.hip", "rhip_raster.hip", "rhip_shade.hip", "rhip_ord1.hip", "rhip_ord4.hip", "rhip_read.hip",
+                   "rhip_batch.hip", "rhip_batch_vis1.hip", "rhip_batch_vis4.hip", "rhip_libm.hip"],
 }
 OBJ_DIR = os.path.join(LIB_DIR, "obj")
 

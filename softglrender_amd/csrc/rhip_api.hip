@@ -169,17 +169,22 @@ constexpr size_t kScratchBytes = (size_t)64 << 20;
 static __device__ __align__(256) char scratch[kScratchBytes];
 
 /* After a synchronisation: reports (RHIP_E_DEVICE, naming the stage) and
- * clears what the kernels' error words recorded since the last check. */
-int takeDeviceErrors(rhip_device d) {
-  uint32_t e[kErrSlots];
-  HIPCHK(hipMemcpy(e, d->errors, sizeof e, hipMemcpyDeviceToHost));
+ * clears what the kernels' error words recorded since the last check; `e` is
+ * the host's copy of them. */
+int reportDeviceErrors(rhip_device d, const uint32_t *e) {
   if (!e[kErrClip]) return RHIP_OK;
-  HIPCHK(hipMemsetAsync(d->errors, 0, sizeof e, d->stream));
+  HIPCHK(hipMemsetAsync(d->errors, 0, kErrSlots * sizeof *e, d->stream));
   HIPCHK(hipStreamSynchronize(d->stream));
   return fail(RHIP_E_DEVICE,
               "clipping: a clipped polygon exceeded %d vertices and its triangle was dropped; the output differs "
               "from the reference's",
               kMaxPoly);
+}
+
+int takeDeviceErrors(rhip_device d) {
+  uint32_t e[kErrSlots];
+  HIPCHK(hipMemcpy(e, d->errors, sizeof e, hipMemcpyDeviceToHost));
+  return reportDeviceErrors(d, e);
 }
 
 __global__ void k_set_error(uint32_t *errors, int slot) { errors[slot] = 1u; }
@@ -507,6 +512,7 @@ int rhip_device_create(int hip_device, rhip_device *out) {
       return rc;
     }
   }
+  readDeviceAdded();
   *out = d.release();
   return RHIP_OK;
 }
@@ -530,6 +536,7 @@ int rhip_device_destroy(rhip_device d) {
     if (p) hipFree(p);
   hipStreamDestroy(d->stream);
   delete d;
+  readDeviceGone();
   return RHIP_OK;
 }
 
@@ -633,29 +640,23 @@ int rhip_texture_read(rhip_device d, int id, int layer, int level, int which, vo
   if (layer < 0 || layer >= t->hd.layers || level < 0 || level >= t->hd.levels)
     return fail(RHIP_E_INVALID, "layer %d / level %d out of range", layer, level);
   const TexLevel &lv = t->hd.lv[layer][level];
+  uint32_t e[kErrSlots];
   if (which == 1) {
     if (!t->desc.multi_sample) return fail(RHIP_E_INVALID, "texture is not multisampled");
     size_t n = (size_t)lv.w * lv.h * 16;
     if (bytes < n) return fail(RHIP_E_INVALID, "output too small");
-    HIPCHK(hipMemcpyAsync(out, t->data + lv.offset, n, hipMemcpyDeviceToHost, d->stream));
-    HIPCHK(hipStreamSynchronize(d->stream));
-    return takeDeviceErrors(d);
+    if ((rc = readLinear(d, t->data + lv.offset, n / 4, out, e))) return rc;
+    return reportDeviceErrors(d, e);
   }
   size_t n = (size_t)lv.w * lv.h * 4;
   if (bytes < n) return fail(RHIP_E_INVALID, "output too small");
   if (t->desc.multi_sample) {
     if (!t->resolved) return fail(RHIP_E_INVALID, "a multisampled depth texture has no single-sample image");
-    HIPCHK(hipMemcpyAsync(out, t->resolved, n, hipMemcpyDeviceToHost, d->stream));
-    HIPCHK(hipStreamSynchronize(d->stream));
-    return takeDeviceErrors(d);
+    if ((rc = readLinear(d, t->resolved, n / 4, out, e))) return rc;
+    return reportDeviceErrors(d, e);
   }
-  std::vector<uint32_t> tmp((size_t)lv.inner_w * lv.inner_h);
-  HIPCHK(hipMemcpyAsync(tmp.data(), t->data + lv.offset, tmp.size() * 4, hipMemcpyDeviceToHost, d->stream));
-  HIPCHK(hipStreamSynchronize(d->stream));
-  uint32_t *o = (uint32_t *)out;
-  for (int y = 0; y < lv.h; y++)
-    for (int x = 0; x < lv.w; x++) o[(size_t)y * lv.w + x] = tmp[hostTexelIndex(lv, t->hd.layout, x, y)];
-  return takeDeviceErrors(d);
+  if ((rc = readLevel(d, t->data + lv.offset, lv, t->hd.layout, out, e))) return rc;
+  return reportDeviceErrors(d, e);
 }
 
 int rhip_texture_destroy(rhip_device d, int id) {

@@ -207,6 +207,14 @@ int libmTableStats(int fn, long long *entries, double *gate);
 /* t[0, 256): powf(k / 255, 2.2); t[256 + k]: smallest c >= 0 whose output byte is at least k. */
 void gammaTablesHost(float *t);
 float hostPowf(float x, float y);
+/* Waits for the stream's work so far and copies a level's image, row-major, to host memory (rhip_read.hip);
+ * `errors` (kErrSlots words, may be null) gets the device's error words. */
+int readLevel(rhip_device d, const uint8_t *src, const TexLevel &lv, int layout, void *out, uint32_t *errors);
+/* The same for `words` 4-byte words of device memory (16-byte aligned). */
+int readLinear(rhip_device d, const void *src, size_t words, void *out, uint32_t *errors);
+/* What the reads share (pinned memory, helper threads) lives while the process has devices. */
+void readDeviceAdded();
+void readDeviceGone();
 /* The IBL shaders' loop tables from the host libm's sinf / cosf. */
 void iblTablesHost(IblTables *t);
 
