@@ -530,9 +530,8 @@ int rhip_device_destroy(rhip_device d) {
   if (d->libm) hipFree(d->libm);
   for (void *p : d->libm_bufs) hipFree(p);
   if (d->errors) hipFree(d->errors);
-  for (void *p : {(void *)d->nn.params, (void *)d->nn.grad, (void *)d->nn.m1, (void *)d->nn.m2, (void *)d->nn.packed,
-                  (void *)d->nn.scratch, (void *)d->nn.hist, (void *)d->nn.rec_count, (void *)d->nn.partial,
-                  (void *)d->nn.lossp})
+  for (void *p : {(void *)d->nn.params, (void *)d->nn.m1, (void *)d->nn.m2, (void *)d->nn.packed, (void *)d->nn.scratch,
+                  (void *)d->nn.rec_count, (void *)d->nn.partial, (void *)d->nn.lossp})
     if (p) hipFree(p);
   hipStreamDestroy(d->stream);
   delete d;
@@ -1152,15 +1151,16 @@ static int nnEnsure(rhip_device d) {
   if (n.params) return RHIP_OK;
   const size_t pb = kNnParams * sizeof(float);
   HIPCHK(hipMalloc(&n.params, pb));
-  HIPCHK(hipMalloc(&n.grad, pb));
   HIPCHK(hipMalloc(&n.m1, pb));
   HIPCHK(hipMalloc(&n.m2, pb));
   HIPCHK(hipMalloc(&n.packed, sizeof(NnPacked)));
   HIPCHK(hipMemsetAsync(n.packed, 0, sizeof(NnPacked), d->stream)); /* padding entries stay zero */
   HIPCHK(hipMalloc(&n.partial, (size_t)kNnMaxParts * kNnParams * sizeof(float)));
   HIPCHK(hipMalloc(&n.lossp, kNnMaxParts * sizeof(double)));
-  HIPCHK(hipMalloc(&n.scratch, 8 * sizeof(double)));
-  HIPCHK(hipMalloc(&n.hist, 2 * kNnHistBins * sizeof(unsigned int)));
+  /* what a gradient or an evaluation gives the host, in one piece (one read) */
+  HIPCHK(hipMalloc(&n.scratch, 8 * sizeof(double) + 2 * kNnHistBins * sizeof(unsigned int) + pb));
+  n.hist = (unsigned int *)(n.scratch + 8);
+  n.grad = (float *)(n.hist + 2 * kNnHistBins);
   HIPCHK(hipMalloc(&n.rec_count, sizeof(unsigned long long)));
   HIPCHK(hipMemsetAsync(n.rec_count, 0, sizeof(unsigned long long), d->stream));
   return RHIP_OK;
@@ -1216,9 +1216,7 @@ int rhip_neural_get_weights(rhip_device d, float *w, int n) {
   if (rc) return rc;
   if (!d->nn.ready) return fail(RHIP_E_INVALID, "learned shader: no network");
   if (!w || n != kNnParams) return fail(RHIP_E_INVALID, "learned shader: %d parameters expected", kNnParams);
-  HIPCHK(hipMemcpyAsync(w, d->nn.params, kNnParams * sizeof(float), hipMemcpyDeviceToHost, d->stream));
-  HIPCHK(hipStreamSynchronize(d->stream));
-  return RHIP_OK;
+  return readLinear(d, d->nn.params, kNnParams, w, nullptr);
 }
 
 int rhip_neural_records(rhip_device d, long long capacity) {
@@ -1312,9 +1310,11 @@ int rhip_neural_gradient(rhip_device d, long long first, int count, float *grad,
   RHIP_LAUNCH(k_nn_update, kNnUpdateBlocks, 256, d->stream, n.params, n.partial, parts, n.lossp, n.scratch, n.grad,
               n.m1, n.m2, n.packed, 0.f, 0.f, 0.f, 0.f, 0.f, 0);
   HIPCHK(hipGetLastError());
-  if (grad) HIPCHK(hipMemcpyAsync(grad, n.grad, kNnParams * sizeof(float), hipMemcpyDeviceToHost, d->stream));
-  if (loss) HIPCHK(hipMemcpyAsync(loss, n.scratch, sizeof(double), hipMemcpyDeviceToHost, d->stream));
-  HIPCHK(hipStreamSynchronize(d->stream));
+  const size_t before = (size_t)((char *)n.grad - (char *)n.scratch);
+  std::vector<char> res(before + kNnParams * sizeof(float));
+  if ((rc = readLinear(d, n.scratch, res.size() / 4, res.data(), nullptr))) return rc;
+  if (grad) memcpy(grad, res.data() + before, kNnParams * sizeof(float));
+  if (loss) memcpy(loss, res.data(), sizeof(double));
   return RHIP_OK;
 }
 
@@ -1326,9 +1326,9 @@ int rhip_neural_train(rhip_device d, long long first, long long count, int steps
   auto &n = d->nn;
   std::vector<double> lh;
   double *dl = nullptr;
-  if (losses && steps > 0) {
-    HIPCHK(hipMalloc(&dl, steps * sizeof(double)));
-    HIPCHK(hipMemsetAsync(dl, 0, steps * sizeof(double), d->stream));
+  if (losses && steps > 0) { /* every step writes its own */
+    if ((rc = n.losses.ensure(steps * sizeof(double)))) return rc;
+    dl = n.losses.as<double>();
   }
   const int grid = std::min<int>((batch + 63) / 64, 512);
   for (int i = 0; i < steps; i++) {
@@ -1346,12 +1346,10 @@ int rhip_neural_train(rhip_device d, long long first, long long count, int steps
   HIPCHK(hipGetLastError());
   if (dl) {
     lh.resize(steps);
-    HIPCHK(hipMemcpyAsync(lh.data(), dl, steps * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-  }
-  HIPCHK(hipStreamSynchronize(d->stream));
-  if (dl) {
-    hipFree(dl);
+    if ((rc = readLinear(d, dl, (size_t)steps * 2, lh.data(), nullptr))) return rc;
     for (int i = 0; i < steps; i++) losses[i] = lh[i] / ((double)batch * kNnOut);
+  } else {
+    HIPCHK(hipStreamSynchronize(d->stream));
   }
   return RHIP_OK;
 }
@@ -1380,20 +1378,25 @@ int rhip_neural_evaluate(rhip_device d, long long first, long long count, int ma
   if (count > INT32_MAX) return fail(RHIP_E_INVALID, "too many records");
   auto &n = d->nn;
   float *dout = nullptr;
-  if (outputs) HIPCHK(hipMalloc(&dout, (size_t)count * 3 * sizeof(float)));
+  if (outputs) {
+    if ((rc = n.outputs.ensure((size_t)count * 3 * sizeof(float)))) return rc;
+    dout = n.outputs.as<float>();
+  }
   HIPCHK(hipMemsetAsync(n.hist, 0, 2 * kNnHistBins * sizeof(unsigned int), d->stream));
   HIPCHK(hipMemsetAsync(n.scratch, 0, 8 * sizeof(double), d->stream));
-  RHIP_LAUNCH(k_nn_eval, (unsigned)std::min<long long>((count + 255) / 256, 2048), 256, d->stream, n.packed,
+  /* two blocks a CU: each adds its histogram to the device's once */
+  RHIP_LAUNCH(k_nn_eval, (unsigned)std::min<long long>((count + 255) / 256, 512), 256, d->stream, n.packed,
               n.records.as<float>(), first, (int)count, material, n.hist, n.hist + kNnHistBins, n.scratch, dout);
   HIPCHK(hipGetLastError());
-  std::vector<unsigned int> h(2 * kNnHistBins);
-  double sums[8];
-  HIPCHK(hipMemcpyAsync(h.data(), n.hist, h.size() * 4, hipMemcpyDeviceToHost, d->stream));
-  HIPCHK(hipMemcpyAsync(sums, n.scratch, sizeof sums, hipMemcpyDeviceToHost, d->stream));
-  if (dout) HIPCHK(hipMemcpyAsync(outputs, dout, (size_t)count * 3 * sizeof(float), hipMemcpyDeviceToHost, d->stream));
-  HIPCHK(hipStreamSynchronize(d->stream));
-  if (dout) hipFree(dout);
-  std::vector<unsigned int> hn(h.begin(), h.begin() + kNnHistBins), hp(h.begin() + kNnHistBins, h.end());
+  struct {
+    double sums[8];
+    unsigned int h[2 * kNnHistBins];
+  } res;
+  if ((rc = readLinear(d, n.scratch, sizeof res / 4, &res, nullptr))) return rc;
+  if (dout && (rc = readLinear(d, dout, (size_t)count * 3, outputs, nullptr))) return rc;
+  const unsigned int *h = res.h;
+  const double *sums = res.sums;
+  std::vector<unsigned int> hn(h, h + kNnHistBins), hp(h + kNnHistBins, h + 2 * kNnHistBins);
   if (nn_err) histStats(hn, sums[0], sums[2], sums[4], nn_err);
   if (plain_err) histStats(hp, sums[1], sums[3], sums[4], plain_err);
   return RHIP_OK;

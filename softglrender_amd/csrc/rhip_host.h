@@ -135,6 +135,8 @@ struct rhip_device_s {
     int step = 0;
     bool ready = false;
     rhip::DevBuf records;
+    rhip::DevBuf outputs; /* an evaluation's network outputs */
+    rhip::DevBuf losses;  /* a training run's, one per step */
     long long rec_cap = 0;
     unsigned long long *rec_count = nullptr;
     bool capturing = false;

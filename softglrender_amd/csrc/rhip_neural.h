@@ -35,16 +35,14 @@ constexpr int kNnUpdateBlocks = (kNnParams + 15) / 16; /* k_nn_update: 16 parame
 
 /* bf16 operands packed for MFMA (device): W1 with b1 in column 24, W2, W3
  * padded to 16 rows, and the transposes backward needs; biases of layers 2, 3.
- * w2r and w3r are W2 and W3 with their columns in the order nnRegUnit gives,
- * for the inference kernel that keeps activations in registers. */
+ * w2r, w3r and w2tr are W2, W3 and W2^T with their columns in the order
+ * nnRegUnit gives, for kernels that keep activations in registers. */
 struct NnPacked {
   __bf16 w1[kNnHid * kNnK1];
-  __bf16 w2[kNnHid * kNnHid];
-  __bf16 w3[16 * kNnHid];
-  __bf16 w2t[kNnHid * kNnHid];
   __bf16 w3t[kNnHid * 32];
   __bf16 w2r[kNnHid * kNnHid];
   __bf16 w3r[16 * kNnHid];
+  __bf16 w2tr[kNnHid * kNnHid];
   float b2[kNnHid];
   float b3[16];
 };
@@ -125,11 +123,6 @@ __device__ __forceinline__ void nnFeatures(f3 N, f3 V, float rough, float metal,
   f[24] = 1.f;
 #pragma unroll
   for (int k = 25; k < kNnK1; k++) f[k] = 0.f;
-}
-
-__device__ __forceinline__ void recFeatures(const float *r, float *f) {
-  nnFeatures({r[kRecN], r[kRecN + 1], r[kRecN + 2]}, {r[kRecV], r[kRecV + 1], r[kRecV + 2]}, r[kRecRough],
-             r[kRecMetal], r[kRecAlbedo], r[kRecAlbedo + 1], r[kRecAlbedo + 2], f);
 }
 
 /* Inference LDS. Rows are padded by 8 bf16 so that the 16 rows one MFMA operand
@@ -610,19 +603,21 @@ __global__ __launch_bounds__(256) void k_nn_eval(const NnPacked *W, const float 
   __shared__ NnWaveLds lds[4];
   __shared__ NnBlockW bw;
   __shared__ unsigned int h_nn[kNnHistBins], h_pl[kNnHistBins];
-  __shared__ double s_sum[6];
+  __shared__ double s_sum[4][5]; /* per wavefront */
   for (int i = threadIdx.x; i < kNnHistBins; i += blockDim.x) h_nn[i] = h_pl[i] = 0;
-  if (threadIdx.x < 6) s_sum[threadIdx.x] = 0;
   nnLoadBlockW(*W, bw);
   __syncthreads();
   NnWaveLds &L = lds[threadIdx.x >> 6];
   double e_nn = 0, e_pl = 0, m_nn = 0, m_pl = 0, n_ok = 0;
   for (int b0 = blockIdx.x * blockDim.x; b0 < count; b0 += gridDim.x * blockDim.x) {
     const int i = b0 + threadIdx.x;
-    const float *r = rec + (size_t)(first + (i < count ? i : 0)) * kRecFloats;
-    const bool act = i < count && (material < 0 || (int)r[kRecMaterial] == material);
+    const float4 *r = (const float4 *)(rec + (size_t)(first + (i < count ? i : 0)) * kRecFloats);
+    const float4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3], r4 = r[4];
+    static_assert(kRecN == 0 && kRecV == 3 && kRecAlbedo == 6 && kRecRough == 10 && kRecMetal == 11 &&
+                      kRecMaterial == 13 && kRecTarget == 14 && kRecPlain == 17, "record layout");
+    const bool act = i < count && (material < 0 || (int)r3.y == material);
     float f[kNnK1];
-    recFeatures(r, f);
+    nnFeatures({r0.x, r0.y, r0.z}, {r0.w, r1.x, r1.y}, r2.z, r2.w, r1.z, r1.w, r2.x, f);
     float y[3];
     nnForward64(bw, L, f, y);
     if (out && i < count) {
@@ -632,10 +627,11 @@ __global__ __launch_bounds__(256) void k_nn_eval(const NnPacked *W, const float 
     }
     if (!act) continue;
     n_ok += 1;
+    const float target[3] = {r3.z, r3.w, r4.x}, plain[3] = {r4.y, r4.z, r4.w};
 #pragma unroll
     for (int ch = 0; ch < 3; ch++) {
-      const float en = fabsf(gclamp(y[ch], 0.f, 1.f) - r[kRecTarget + ch]) * 255.f;
-      const float ep = fabsf(r[kRecPlain + ch] - r[kRecTarget + ch]) * 255.f;
+      const float en = fabsf(gclamp(y[ch], 0.f, 1.f) - target[ch]) * 255.f;
+      const float ep = fabsf(plain[ch] - target[ch]) * 255.f;
       atomicAdd(&h_nn[histBin(en)], 1u);
       atomicAdd(&h_pl[histBin(ep)], 1u);
       e_nn += en;
@@ -644,39 +640,62 @@ __global__ __launch_bounds__(256) void k_nn_eval(const NnPacked *W, const float 
       m_pl = fmax(m_pl, (double)ep);
     }
   }
-  atomicAdd(&s_sum[0], e_nn);
-  atomicAdd(&s_sum[1], e_pl);
-  atomicAdd(&s_sum[4], n_ok);
+  /* sums and maxima: lanes, then wavefronts, then one atomic each per block (an atomic per thread on the same
+   * addresses took most of the kernel's time) */
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    e_nn += __shfl_xor(e_nn, o, 64);
+    e_pl += __shfl_xor(e_pl, o, 64);
+    n_ok += __shfl_xor(n_ok, o, 64);
+    m_nn = fmax(m_nn, __shfl_xor(m_nn, o, 64));
+    m_pl = fmax(m_pl, __shfl_xor(m_pl, o, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    double *t = s_sum[threadIdx.x >> 6];
+    t[0] = e_nn, t[1] = e_pl, t[2] = m_nn, t[3] = m_pl, t[4] = n_ok;
+  }
   __syncthreads();
   for (int i = threadIdx.x; i < kNnHistBins; i += blockDim.x) {
     if (h_nn[i]) atomicAdd(&hist_nn[i], h_nn[i]);
     if (h_pl[i]) atomicAdd(&hist_plain[i], h_pl[i]);
   }
-  if (threadIdx.x == 0) {
-    atomicAdd(&sums[0], s_sum[0]);
-    atomicAdd(&sums[1], s_sum[1]);
-    atomicAdd(&sums[4], s_sum[4]);
+  if (threadIdx.x < 5) {
+    const int k = threadIdx.x;
+    const double a = s_sum[0][k], b = s_sum[1][k], c = s_sum[2][k], d = s_sum[3][k];
+    if (k == 2 || k == 3) /* through the integer bits of non-negative doubles */
+      atomicMax((unsigned long long *)&sums[k],
+                (unsigned long long)__double_as_longlong(fmax(fmax(a, b), fmax(c, d))));
+    else
+      atomicAdd(&sums[k], (a + b) + (c + d));
   }
-  /* maxima: through the integer bits of non-negative doubles */
-  atomicMax((unsigned long long *)&sums[2], (unsigned long long)__double_as_longlong(m_nn));
-  atomicMax((unsigned long long *)&sums[3], (unsigned long long)__double_as_longlong(m_pl));
 }
 
 /* --------------------------------------------------------------------------- training */
 
-/* Per-wavefront LDS of one training chunk (64 fragments). */
+/* One chunk (64 records) of a training step: what the gradient products contract
+ * over the records, as [unit or feature][record] rows, padded so that the 16 rows
+ * an operand load touches start in different banks. */
+constexpr int kTs = 64 + 8;
 struct NnTrainLds {
-  __bf16 x[64 * kNnK1];    /* X[frag][feat] */
-  __bf16 xt[kNnK1 * 64];   /* X^T[feat][frag] */
-  __bf16 h1[64 * kNnHid];  /* H1[frag][unit] */
-  __bf16 h1t[kNnHid * 64]; /* H1^T, later dH1^T */
-  __bf16 h2[64 * kNnHid];  /* H2, later dH2[frag][unit] */
-  __bf16 h2t[kNnHid * 64]; /* H2^T, later dH2^T */
-  __bf16 dy[64 * 32];      /* dY[frag][channel] (3 used) */
-  __bf16 dyt[16 * 64];     /* dY^T[channel][frag] */
-  float yf[64 * 4];        /* outputs of the chunk */
-  float g[kNnParams];      /* gradient sums of this block */
+  __bf16 xt[kNnK1 * kTs];
+  __bf16 h1t[kNnHid * kTs];
+  __bf16 h2t[kNnHid * kTs];
+  __bf16 dh1t[kNnHid * kTs];
+  __bf16 dh2t[kNnHid * kTs];
+  __bf16 dyt[16 * kTs];
+  double loss[64];
 };
+
+/* reluPack that keeps NaN, so that a run that diverges shows it */
+__device__ __forceinline__ bf16x8 reluPackNan(f32x4 lo, f32x4 hi) {
+  bf16x8 o;
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    o[v] = (__bf16)gmax(lo[v], 0.f);
+    o[4 + v] = (__bf16)gmax(hi[v], 0.f);
+  }
+  return o;
+}
 
 /* sum over the 16 rows of a product tile: MFMA with an all-ones operand */
 __device__ __forceinline__ bf16x8 onesOp() {
@@ -688,214 +707,159 @@ __device__ __forceinline__ bf16x8 onesOp() {
 
 /* One training step's gradient of mean squared error over `batch` records
  * drawn from [first, first + count) (or the `batch` records starting at
- * `first` when `count` is 0): forward and backward on MFMA, gradients summed
- * per block in LDS. A block takes chunks of 64 records with four wavefronts:
- * wavefront w computes the output tiles of hidden units 16w..16w+15 of every
- * layer (and fragment tile w where a layer has one row tile), so each gradient
- * sum has one writer and the same order as with one wavefront; wavefront 0
- * stages the records and takes their errors. Each block writes its sums (FP32,
- * unscaled) to its own row of `partial` and its squared error to
- * lossp[block]: no atomics, so k_nn_update's fixed-order sum makes a step
- * reproducible bit for bit. */
+ * `first` when `count` is 0). A block takes chunks of 64 records: each of its
+ * four wavefronts runs 16 of them forward and backward with the activations in
+ * registers (every layer's result tiles are the next one's operand, as in
+ * nnLayers), and leaves activations and their gradients in LDS transposed;
+ * then wavefront w multiplies out the gradients of hidden units 16w..16w+15
+ * (and unit tile w of W3), summed over its chunks in registers. Latency bounds
+ * it (a step is one chunk a block, a chain of five products and the record
+ * gather): two barriers a chunk. With every layer's tiles exchanged through
+ * LDS, ten barriers and 70 KB of it, 16,384 records took 16.3 us (now 12.3) and
+ * 300,007 128 us (74).
+ * Each block writes its sums (FP32, unscaled) to its own row of `partial` and
+ * its squared error to lossp[block]: no atomics, so k_nn_update's fixed-order
+ * sum makes a step reproducible bit for bit. */
 constexpr int kNnGradThreads = 256;
 __global__ __launch_bounds__(kNnGradThreads) void k_nn_grad(const NnPacked *W, const float *rec, long long first,
                                                             long long count, int batch, uint32_t seed,
                                                             float *partial, double *lossp) {
   __shared__ NnTrainLds L;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, c = l & 15;
-  const int m = w; /* this wavefront's row tile of the hidden layers */
-  for (int i = threadIdx.x; i < kNnParams; i += kNnGradThreads) L.g[i] = 0.f;
+  const int fr = 16 * w + c; /* this lane's record of the chunk */
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 gw2[4], gw1[2], gw3 = zero, gb2 = zero, gb3 = zero;
+#pragma unroll
+  for (int n = 0; n < 4; n++) gw2[n] = zero;
+#pragma unroll
+  for (int n = 0; n < 2; n++) gw1[n] = zero;
   double lsum = 0;
   const bf16x8 ones = onesOp();
   for (int c0 = blockIdx.x * 64; c0 < batch; c0 += gridDim.x * 64) {
-    const int bi = c0 + l;
+    const int bi = c0 + fr;
     const bool act = bi < batch;
     long long ri = first + bi;
     if (count > 0) ri = first + (long long)(hash32((uint32_t)bi * 0x9e3779b9u ^ seed) % (uint32_t)count);
-    const float *r = rec + (size_t)(act ? ri : first) * kRecFloats;
-    if (w == 0) {
+    const float4 *r = (const float4 *)(rec + (size_t)(act ? ri : first) * kRecFloats);
+    const float4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3], r4 = r[4];
+    static_assert(kRecN == 0 && kRecV == 3 && kRecAlbedo == 6 && kRecRough == 10 && kRecMetal == 11 && kRecTarget == 14,
+                  "record layout");
+    bf16x8 xb;
+    {
       float f[kNnK1];
-      recFeatures(r, f);
-      if (!act) {
+      nnFeatures({r0.x, r0.y, r0.z}, {r0.w, r1.x, r1.y}, r2.z, r2.w, r1.z, r1.w, r2.x, f);
 #pragma unroll
-        for (int k = 0; k < kNnK1; k++) f[k] = 0.f;
-      }
-#pragma unroll
-      for (int k = 0; k < kNnK1; k++) {
-        L.x[l * kNnK1 + k] = (__bf16)f[k];
-        L.xt[k * 64 + l] = (__bf16)f[k];
+      for (int k = 0; k < 8; k++) {
+        const float v = g == 0 ? f[k] : g == 1 ? f[8 + k] : g == 2 ? f[16 + k] : f[24 + k];
+        xb[k] = (__bf16)(act ? v : 0.f);
+        L.xt[(8 * g + k) * kTs + fr] = xb[k];
       }
     }
-    __syncthreads();
-    /* forward: H1, H2 (and transposes), Y */
-    {
-      const bf16x8 a = ldOp(W->w1, kNnK1, 16 * m, 0);
+    /* forward; lane (g, c) holds units 16m + 4g + v of record c */
+    f32x4 h1[4], h2[4];
+    bf16x8 b1[2], b2[2];
 #pragma unroll
-      for (int n = 0; n < 4; n++) {
-        f32x4 d = {0.f, 0.f, 0.f, 0.f};
-        d = mma16(a, ldOp(L.x, kNnK1, 16 * n, 0), d);
+    for (int kb = 0; kb < 2; kb++) {
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const __bf16 h = (__bf16)gmax(d[v], 0.f);
-          const int u = 16 * m + 4 * g + v, fr = 16 * n + c;
-          L.h1[fr * kNnHid + u] = h;
-          L.h1t[u * 64 + fr] = h;
-        }
-      }
+      for (int t = 0; t < 2; t++) h1[2 * kb + t] = mma16(ldOp(W->w1, kNnK1, 32 * kb + 16 * t, 0), xb, zero);
+      b1[kb] = reluPackNan(h1[2 * kb], h1[2 * kb + 1]);
     }
-    __syncthreads();
-    {
-      const bf16x8 a0 = ldOp(W->w2, kNnHid, 16 * m, 0), a1 = ldOp(W->w2, kNnHid, 16 * m, 32);
-      f32x4 bias;
 #pragma unroll
-      for (int v = 0; v < 4; v++) bias[v] = W->b2[16 * m + 4 * g + v];
+    for (int kb = 0; kb < 2; kb++) {
 #pragma unroll
-      for (int n = 0; n < 4; n++) {
-        const f32x4 d = mma16(a1, ldOp(L.h1, kNnHid, 16 * n, 32), mma16(a0, ldOp(L.h1, kNnHid, 16 * n, 0), bias));
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const __bf16 h = (__bf16)gmax(d[v], 0.f);
-          const int u = 16 * m + 4 * g + v, fr = 16 * n + c;
-          L.h2[fr * kNnHid + u] = h;
-          L.h2t[u * 64 + fr] = h;
-        }
+      for (int t = 0; t < 2; t++) {
+        const int m = 2 * kb + t;
+        const f32x4 bias = *(const f32x4 *)&W->b2[16 * m + 4 * g];
+        h2[m] = mma16(ldOp(W->w2r, kNnHid, 16 * m, 32), b1[1], mma16(ldOp(W->w2r, kNnHid, 16 * m, 0), b1[0], bias));
       }
+      b2[kb] = reluPackNan(h2[2 * kb], h2[2 * kb + 1]);
     }
-    __syncthreads();
-    {
-      const bf16x8 a0 = ldOp(W->w3, kNnHid, 0, 0), a1 = ldOp(W->w3, kNnHid, 0, 32);
-      f32x4 bias;
+    const f32x4 y = mma16(ldOp(W->w3r, kNnHid, 0, 32), b2[1],
+                          mma16(ldOp(W->w3r, kNnHid, 0, 0), b2[0], *(const f32x4 *)&W->b3[4 * g]));
+    /* the error: lanes 0..15 hold their record's channels; dY's operand has the channels as K */
+    bf16x8 dy;
 #pragma unroll
-      for (int v = 0; v < 4; v++) bias[v] = W->b3[4 * g + v];
-      const int n = w, fr = 16 * n + c;
-      const f32x4 d = mma16(a1, ldOp(L.h2, kNnHid, 16 * n, 32), mma16(a0, ldOp(L.h2, kNnHid, 16 * n, 0), bias));
-      if (g == 0) {
-#pragma unroll
-        for (int v = 0; v < 4; v++) L.yf[fr * 4 + v] = d[v];
-      }
-    }
-    __syncthreads();
-    /* record l's error and dY (wavefront 0) */
-    if (w == 0) {
-      float dyv[3];
+    for (int k = 0; k < 8; k++) dy[k] = (__bf16)0.f;
+    if (g == 0) {
+      const float tgt[3] = {r3.z, r3.w, r4.x};
 #pragma unroll
       for (int ch = 0; ch < 3; ch++) {
-        const float y = L.yf[l * 4 + ch];
-        const float e = act ? y - r[kRecTarget + ch] : 0.f;
+        const float e = act ? y[ch] - tgt[ch] : 0.f;
         lsum += (double)e * e;
-        dyv[ch] = 2.f * e;
+        dy[ch] = (__bf16)(2.f * e);
       }
-#pragma unroll
-      for (int ch = 0; ch < 32; ch++) L.dy[l * 32 + ch] = (__bf16)(ch < 3 ? dyv[ch] : 0.f);
-#pragma unroll
-      for (int ch = 0; ch < 16; ch++) L.dyt[ch * 64 + l] = (__bf16)(ch < 3 ? dyv[ch] : 0.f);
     }
-    __syncthreads();
-    /* dW3 = dY^T . H2 (unit tile w), db3 = row sums of dY^T (wavefront 0) */
-    {
-      const bf16x8 a0 = ldOp(L.dyt, 64, 0, 0), a1 = ldOp(L.dyt, 64, 0, 32);
-      const int n = w;
-      f32x4 d = {0.f, 0.f, 0.f, 0.f};
-      d = mma16(a1, ldOp(L.h2t, 64, 16 * n, 32), mma16(a0, ldOp(L.h2t, 64, 16 * n, 0), d));
+#pragma unroll
+    for (int v = 0; v < 4; v++) L.dyt[(4 * g + v) * kTs + fr] = g == 0 ? dy[v] : (__bf16)0.f;
+    /* backward: dH2 = W3^T dY where H2 > 0, dH1 = W2^T dH2 where H1 > 0. A unit is on when its bf16 value is. */
+    f32x4 d2[4];
+    bf16x8 bd[2];
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      d2[m] = mma16(ldOp(W->w3t, 32, 16 * m, 0), dy, zero);
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        const int ch = 4 * g + v;
-        if (ch < kNnOut) L.g[kOffW3 + ch * kNnHid + 16 * n + c] += d[v];
-      }
-      if (w == 0) {
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
-        s = mma16(a1, ones, mma16(a0, ones, s));
-        if (c == 0) {
-#pragma unroll
-          for (int v = 0; v < 4; v++)
-            if (4 * g + v < kNnOut) L.g[kOffB3 + 4 * g + v] += s[v];
-        }
+        const int u = 16 * m + 4 * g + v;
+        const __bf16 a1 = b1[m >> 1][4 * (m & 1) + v], a2 = b2[m >> 1][4 * (m & 1) + v];
+        const __bf16 dh = (__bf16)((float)a2 > 0.f ? d2[m][v] : 0.f);
+        bd[m >> 1][4 * (m & 1) + v] = dh;
+        L.h1t[u * kTs + fr] = a1;
+        L.h2t[u * kTs + fr] = a2;
+        L.dh2t[u * kTs + fr] = dh;
       }
     }
-    __syncthreads(); /* H2^T is read above before it is overwritten below */
-    /* dH2^T = W3^T . dY^T, masked by H2 > 0, written over H2 and H2^T */
-    {
-      bf16x8 bdy[4];
 #pragma unroll
-      for (int n = 0; n < 4; n++) bdy[n] = ldOp(L.dy, 32, 16 * n, 0);
-      const bf16x8 a = ldOp(W->w3t, 32, 16 * m, 0);
+    for (int m = 0; m < 4; m++) {
+      const f32x4 d1 = mma16(ldOp(W->w2tr, kNnHid, 16 * m, 32), bd[1], mma16(ldOp(W->w2tr, kNnHid, 16 * m, 0), bd[0], zero));
 #pragma unroll
-      for (int n = 0; n < 4; n++) {
-        f32x4 d = {0.f, 0.f, 0.f, 0.f};
-        d = mma16(a, bdy[n], d);
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int u = 16 * m + 4 * g + v, fr = 16 * n + c;
-          const bool on = (float)L.h2t[u * 64 + fr] > 0.f;
-          const __bf16 dh = (__bf16)(on ? d[v] : 0.f);
-          L.h2t[u * 64 + fr] = dh;
-          L.h2[fr * kNnHid + u] = dh;
-        }
-      }
+      for (int v = 0; v < 4; v++)
+        L.dh1t[(16 * m + 4 * g + v) * kTs + fr] =
+            (__bf16)((float)b1[m >> 1][4 * (m & 1) + v] > 0.f ? d1[v] : 0.f);
     }
     __syncthreads();
-    /* dW2 = dH2^T . H1, db2 = row sums of dH2^T */
     {
-      const bf16x8 a0 = ldOp(L.h2t, 64, 16 * m, 0), a1 = ldOp(L.h2t, 64, 16 * m, 32);
-#pragma unroll
-      for (int n = 0; n < 4; n++) {
-        f32x4 d = {0.f, 0.f, 0.f, 0.f};
-        d = mma16(a1, ldOp(L.h1t, 64, 16 * n, 32), mma16(a0, ldOp(L.h1t, 64, 16 * n, 0), d));
-#pragma unroll
-        for (int v = 0; v < 4; v++) L.g[kOffW2 + (16 * m + 4 * g + v) * kNnHid + 16 * n + c] += d[v];
-      }
-      f32x4 s = {0.f, 0.f, 0.f, 0.f};
-      s = mma16(a1, ones, mma16(a0, ones, s));
-      if (c == 0) {
-#pragma unroll
-        for (int v = 0; v < 4; v++) L.g[kOffB2 + 16 * m + 4 * g + v] += s[v];
-      }
-    }
-    __syncthreads(); /* H1^T is read above before it is overwritten below */
-    /* dH1^T = W2^T . dH2^T, masked by H1 > 0, written over H1^T */
-    {
-      bf16x8 bd[4][2];
+      /* dW3 = dY^T . H2 (unit tile w), db3 = row sums of dY^T */
+      const bf16x8 y0 = ldOp(L.dyt, kTs, 0, 0), y1 = ldOp(L.dyt, kTs, 0, 32);
+      gw3 += mma16(y1, ldOp(L.h2t, kTs, 16 * w, 32), mma16(y0, ldOp(L.h2t, kTs, 16 * w, 0), zero));
+      gb3 += mma16(y1, ones, mma16(y0, ones, zero));
+      /* dW2 = dH2^T . H1, db2 = row sums of dH2^T (unit rows of tile w) */
+      const bf16x8 a0 = ldOp(L.dh2t, kTs, 16 * w, 0), a1 = ldOp(L.dh2t, kTs, 16 * w, 32);
 #pragma unroll
       for (int n = 0; n < 4; n++)
+        gw2[n] += mma16(a1, ldOp(L.h1t, kTs, 16 * n, 32), mma16(a0, ldOp(L.h1t, kTs, 16 * n, 0), zero));
+      gb2 += mma16(a1, ones, mma16(a0, ones, zero));
+      /* dW1 (with db1 in column 24) = dH1^T . X */
+      const bf16x8 e0 = ldOp(L.dh1t, kTs, 16 * w, 0), e1 = ldOp(L.dh1t, kTs, 16 * w, 32);
 #pragma unroll
-        for (int kb = 0; kb < 2; kb++) bd[n][kb] = ldOp(L.h2, kNnHid, 16 * n, 32 * kb);
-      const bf16x8 a0 = ldOp(W->w2t, kNnHid, 16 * m, 0), a1 = ldOp(W->w2t, kNnHid, 16 * m, 32);
-#pragma unroll
-      for (int n = 0; n < 4; n++) {
-        f32x4 d = {0.f, 0.f, 0.f, 0.f};
-        d = mma16(a1, bd[n][1], mma16(a0, bd[n][0], d));
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int u = 16 * m + 4 * g + v, fr = 16 * n + c;
-          const bool on = (float)L.h1t[u * 64 + fr] > 0.f;
-          L.h1t[u * 64 + fr] = (__bf16)(on ? d[v] : 0.f);
-        }
-      }
+      for (int n = 0; n < 2; n++)
+        gw1[n] += mma16(e1, ldOp(L.xt, kTs, 16 * n, 32), mma16(e0, ldOp(L.xt, kTs, 16 * n, 0), zero));
     }
-    __syncthreads();
-    /* dW1 (with db1 in column 24) = dH1^T . X */
-    {
-      const bf16x8 a0 = ldOp(L.h1t, 64, 16 * m, 0), a1 = ldOp(L.h1t, 64, 16 * m, 32);
-#pragma unroll
-      for (int n = 0; n < 2; n++) {
-        f32x4 d = {0.f, 0.f, 0.f, 0.f};
-        d = mma16(a1, ldOp(L.xt, 64, 16 * n, 32), mma16(a0, ldOp(L.xt, 64, 16 * n, 0), d));
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int u = 16 * m + 4 * g + v, k = 16 * n + c;
-          if (k < kNnIn)
-            L.g[kOffW1 + u * kNnIn + k] += d[v];
-          else if (k == kNnIn)
-            L.g[kOffB1 + u] += d[v];
-        }
-      }
-    }
-    __syncthreads(); /* the chunk's tiles are read before the next chunk overwrites them */
+    __syncthreads(); /* the chunk's rows are read before the next chunk overwrites them */
   }
   float *dst = partial + (size_t)blockIdx.x * kNnParams;
-  for (int i = threadIdx.x; i < kNnParams; i += kNnGradThreads) dst[i] = L.g[i];
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    const int u = 16 * w + 4 * g + v, ch = 4 * g + v;
+#pragma unroll
+    for (int n = 0; n < 4; n++) dst[kOffW2 + u * kNnHid + 16 * n + c] = gw2[n][v];
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+      const int k = 16 * n + c;
+      if (k < kNnIn)
+        dst[kOffW1 + u * kNnIn + k] = gw1[n][v];
+      else if (k == kNnIn)
+        dst[kOffB1 + u] = gw1[n][v];
+    }
+    if (ch < kNnOut) dst[kOffW3 + ch * kNnHid + 16 * w + c] = gw3[v];
+    if (c == 0) {
+      dst[kOffB2 + u] = gb2[v];
+      if (w == 0 && ch < kNnOut) dst[kOffB3 + ch] = gb3[v];
+    }
+  }
+  if (g == 0) L.loss[fr] = lsum;
+  __syncthreads();
   if (w == 0) {
-    double t = lsum;
+    double t = L.loss[l];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
     if (l == 0) lossp[blockIdx.x] = t;
@@ -912,14 +876,12 @@ __device__ __forceinline__ void nnPackParam(NnPacked *W, int i, float x) {
     W->w1[(i - kOffB1) * kNnK1 + kNnIn] = h;
   } else if (i < kOffB2) {
     const int j = i - kOffW2, u = j / kNnHid, k = j % kNnHid;
-    W->w2[j] = h;
-    W->w2t[k * kNnHid + u] = h;
     W->w2r[u * kNnHid + nnRegSlot(k)] = h;
+    W->w2tr[k * kNnHid + nnRegSlot(u)] = h;
   } else if (i < kOffW3) {
     W->b2[i - kOffB2] = x;
   } else if (i < kOffB3) {
     const int j = i - kOffW3, ch = j / kNnHid, k = j % kNnHid;
-    W->w3[j] = h;
     W->w3t[k * 32 + ch] = h;
     W->w3r[ch * kNnHid + nnRegSlot(k)] = h;
   } else {
@@ -929,12 +891,12 @@ __device__ __forceinline__ void nnPackParam(NnPacked *W, int i, float x) {
 
 /* The gradient of a step: the `nparts` block sums of k_nn_grad added in a
  * fixed order (16 interleaved partial sums per parameter, each over batches of
- * 8 independent loads, then those 16 in order), and the loss by a fixed tree.
+ * 16 independent loads, then those 16 in order), and the loss by a fixed tree.
  * With `gout` the gradient is only written there. Otherwise Adam (step > 0)
  * updates the FP32 parameters with the gradient scaled by `scale`, and every
  * parameter is repacked into the bf16 operands (step 0: repack only).
  * kNnUpdateParams parameters per block of 256 threads. */
-constexpr int kNnUpdateSlices = 16, kNnUpdateParams = 256 / kNnUpdateSlices;
+constexpr int kNnUpdateSlices = 16, kNnUpdateParams = 256 / kNnUpdateSlices, kNnUpdateLoads = 16;
 static_assert(kNnUpdateParams == 16 && kNnUpdateBlocks * kNnUpdateParams >= kNnParams, "k_nn_update grid");
 __global__ __launch_bounds__(256) void k_nn_update(float *p, const float *partial, int nparts, const double *lossp,
                                                    double *loss, float *gout, float *m1, float *m2, NnPacked *W,
@@ -943,37 +905,42 @@ __global__ __launch_bounds__(256) void k_nn_update(float *p, const float *partia
   __shared__ double lpart[256];
   const int t = threadIdx.x % kNnUpdateParams, s = threadIdx.x / kNnUpdateParams;
   const int i = blockIdx.x * kNnUpdateParams + t;
+  const bool mine = s == 0 && i < kNnParams, adam = mine && !gout && step > 0;
+  /* what the update needs besides the sums, on its way while they are added */
+  const float p0 = mine && !gout ? p[i] : 0.f, m0 = adam ? m1[i] : 0.f, v0 = adam ? m2[i] : 0.f;
   float acc = 0.f;
   if (i < kNnParams) {
-    for (int b0 = s; b0 < nparts; b0 += 8 * kNnUpdateSlices) {
-      float v[8];
+    for (int b0 = s; b0 < nparts; b0 += kNnUpdateLoads * kNnUpdateSlices) {
+      float v[kNnUpdateLoads];
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
+      for (int j = 0; j < kNnUpdateLoads; j++) {
         const int b = b0 + j * kNnUpdateSlices;
         v[j] = b < nparts ? partial[(size_t)b * kNnParams + i] : 0.f;
       }
 #pragma unroll
-      for (int j = 0; j < 8; j++) acc += v[j];
+      for (int j = 0; j < kNnUpdateLoads; j++) acc += v[j];
     }
   }
+  const float c1 = adam ? 1.f - powf(b1, (float)step) : 0.f, c2 = adam ? 1.f - powf(b2, (float)step) : 0.f;
   part[s][t] = acc;
   __syncthreads();
-  if (s == 0 && i < kNnParams) {
+  if (mine) {
     float gs = 0.f;
 #pragma unroll
     for (int k = 0; k < kNnUpdateSlices; k++) gs += part[k][t];
     if (gout) {
       gout[i] = gs;
     } else {
+      float x = p0;
       if (step > 0) {
-        const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
         const float gi = gs * scale;
-        const float a = b1 * m1[i] + (1.f - b1) * gi, b = b2 * m2[i] + (1.f - b2) * gi * gi;
+        const float a = b1 * m0 + (1.f - b1) * gi, b = b2 * v0 + (1.f - b2) * gi * gi;
         m1[i] = a;
         m2[i] = b;
-        p[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+        x -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+        p[i] = x;
       }
-      nnPackParam(W, i, p[i]);
+      nnPackParam(W, i, x);
     }
   }
   if (loss && blockIdx.x == 0) {
