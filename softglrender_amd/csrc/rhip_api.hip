@@ -859,13 +859,10 @@ int drawPointsLines(rhip_device d, DrawParams &P, const DrawShape &sh, bool no_a
   const bool has_colour = P.color != nullptr;
   const bool points = P.st.primitiveType == 0 || (P.st.primitiveType == 2 && P.st.polygonMode == 0);
   if (U > (long long)INT32_MAX) return fail(RHIP_E_UNSUPPORTED, "draw too large (%lld points or lines)", U);
-  /* phase 1: vertices, units, per-unit counts and offsets, the point sort */
-  size_t sort_tmp = 0, scan_tmp = 0;
-  if (points)
-    HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_tmp, (uint32_t *)nullptr, (uint32_t *)nullptr,
-                                              (uint32_t *)nullptr, (uint32_t *)nullptr, (int)U, 0, 32, s));
+  /* phase 1: vertices, units, per-unit counts and offsets */
+  size_t scan_tmp = 0;
   HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, scan_tmp, (unsigned long long *)nullptr,
-                                          (unsigned long long *)nullptr, (int)U, s));
+                                          (unsigned long long *)nullptr, (size_t)U + 1, s));
   size_t off = 0;
   char *base = nullptr;
   auto take = [&](size_t bytes) {
@@ -875,7 +872,7 @@ int drawPointsLines(rhip_device d, DrawParams &P, const DrawShape &sh, bool no_a
   };
   PlUnit *units = nullptr;
   unsigned long long *count = nullptr, *offset = nullptr;
-  uint32_t *pkey = nullptr, *pval = nullptr, *skey = nullptr, *sval = nullptr;
+  int *head = nullptr, *next = nullptr; /* per vertex, its point units (a linked list) */
   void *tmp = nullptr;
   for (int pass = 0; pass < 2; pass++) {
     off = 0;
@@ -884,13 +881,11 @@ int drawPointsLines(rhip_device d, DrawParams &P, const DrawShape &sh, bool no_a
     P.mask = (int *)take((size_t)V * 4);
     P.vary = (float *)take((size_t)V * P.vary_stride * 4);
     units = (PlUnit *)take((size_t)U * sizeof(PlUnit));
-    count = (unsigned long long *)take((size_t)U * 8);
-    offset = (unsigned long long *)take((size_t)U * 8);
-    pkey = (uint32_t *)take((size_t)U * 4);
-    pval = (uint32_t *)take((size_t)U * 4);
-    skey = (uint32_t *)take((size_t)U * 4);
-    sval = (uint32_t *)take((size_t)U * 4);
-    tmp = take(std::max(sort_tmp, scan_tmp));
+    count = (unsigned long long *)take((size_t)(U + 1) * 8);
+    offset = (unsigned long long *)take((size_t)(U + 1) * 8);
+    head = (int *)take((size_t)V * 4);
+    next = (int *)take((size_t)U * 4);
+    tmp = take(scan_tmp);
     if (pass == 0) {
       int rc = d->arena.ensure(off);
       if (rc) return rc;
@@ -901,20 +896,23 @@ int drawPointsLines(rhip_device d, DrawParams &P, const DrawShape &sh, bool no_a
   unsigned long long total = 0;
   if (U > 0) {
     const unsigned g = blocks((size_t)U, 256);
-    { Timer tm(d, "k_pl_units"); RHIP_LAUNCH(k_pl_units, g, 256, s, P, units, U, count, pkey, pval, has_colour ? 1 : 0); }
+    if (points)
+      RHIP_LAUNCH(k_fill2_u32, std::min(blocks((size_t)V, 1024), 1024u), 256, s, (uint32_t *)head, (size_t)V, 0xffffffffu,
+                  (uint32_t *)nullptr, (size_t)0, 0u);
+    {
+      Timer tm(d, "k_pl_units");
+      RHIP_LAUNCH(k_pl_units, blocks((size_t)U + 1, 256), 256, s, P, units, U, count, head, next, has_colour ? 1 : 0);
+    }
     if (points) {
-      size_t t = sort_tmp;
-      HIPCHK(hipcub::DeviceRadixSort::SortPairs(tmp, t, pkey, skey, pval, sval, (int)U, 0, 32, s));
       Timer tm(d, "k_pl_points");
-      RHIP_LAUNCH(k_pl_points, g, 256, s, P, units, skey, sval, U, count, has_colour ? 1 : 0);
+      RHIP_LAUNCH(k_pl_points, g, 256, s, P, units, head, next, U, count, has_colour ? 1 : 0);
     }
     size_t t = scan_tmp;
-    HIPCHK(hipcub::DeviceScan::ExclusiveSum(tmp, t, count, offset, (int)U, s));
-    unsigned long long last[2] = {0, 0};
-    HIPCHK(hipMemcpyAsync(&last[0], offset + (U - 1), 8, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(&last[1], count + (U - 1), 8, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    total = last[0] + last[1];
+    HIPCHK(hipcub::DeviceScan::ExclusiveSum(tmp, t, count, offset, (size_t)U + 1, s));
+    unsigned long long last[2]; /* 16-byte aligned words that hold offset[U] */
+    int rc = readLinear(d, offset + (U & ~1ll), (U & 1) ? 4 : 2, last, nullptr);
+    if (rc) return rc;
+    total = last[U & 1];
   }
   HIPCHK(hipGetLastError());
   if (total > (unsigned long long)INT32_MAX)
@@ -946,7 +944,7 @@ int drawPointsLines(rhip_device d, DrawParams &P, const DrawShape &sh, bool no_a
       key2 = (uint32_t *)ftake((size_t)F * 4);
       val2 = (uint32_t *)ftake((size_t)F * 4);
       zf = (float *)ftake((size_t)F * 4);
-      cf = (float4 *)ftake((size_t)F * 16);
+      cf = P.shading == RHS_SHADING_BASIC ? nullptr : (float4 *)ftake((size_t)F * 16);
       ftmp = ftake(fsort_tmp);
       if (pass == 0) {
         int rc = d->lines.ensure(foff);
@@ -954,7 +952,7 @@ int drawPointsLines(rhip_device d, DrawParams &P, const DrawShape &sh, bool no_a
         fb = d->lines.as<char>();
       }
     }
-    const unsigned g = blocks((size_t)U, 256), gf = blocks((size_t)F, 256);
+    const unsigned g = std::min(blocks((size_t)U, 16), 1u << 20), gf = blocks((size_t)F, 256);
     { Timer tm(d, "k_pl_emit"); RHIP_LAUNCH(k_pl_emit, g, 256, s, P, units, U, offset, key, val, zf, cf); }
     size_t t = fsort_tmp;
     HIPCHK(hipcub::DeviceRadixSort::SortPairs(ftmp, t, key, key2, val, val2, (int)F, 0, bits, s));
