@@ -59,16 +59,7 @@ static __global__ __launch_bounds__(256) void kb_setup(const DrawParams *__restr
 
 static __global__ __launch_bounds__(256) void kb_clip(const DrawParams *__restrict__ Pv, const uint32_t *__restrict__ tab) {
   const ViewBlock vb = viewBlock(Pv, tab);
-  clipBody(*vb.P, vb.local);
-}
-
-/* one block per view */
-static __global__ __launch_bounds__(1024) void kb_scan_fans(const DrawParams *__restrict__ Pv) { scanFansBody(Pv[blockIdx.x]); }
-
-static __global__ __launch_bounds__(256) void kb_clip_fans(const DrawParams *__restrict__ Pv,
-                                                    const uint32_t *__restrict__ tab) {
-  const ViewBlock vb = viewBlock(Pv, tab);
-  clipFansBody<false>(*vb.P, vb.local);
+  clipBody(*vb.P, vb.local, vb.P->nblk);
 }
 
 /* one block per view */

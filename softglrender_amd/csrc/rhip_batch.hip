@@ -165,13 +165,14 @@ int buildBatch(rhip_device d, Batch &b, const rhip_batch_config &c) {
     b.vao_refs.push_back({dd.vao, d->vao[dd.vao]->verts});
   }
 
-  /* fill ranges: per view its bins and the clears, then the batch counters */
+  /* fill ranges: per view its bins, scalars and clears, then the batch counters */
   const BatchMisc M(nv);
   if ((rc = b.misc.ensure(M.bytes))) return rc;
   char *misc = b.misc.as<char>();
   std::vector<FillRange> fills;
   for (int v = 0; v < nv; v++) {
     fills.push_back({(uint32_t *)P[v].bin_count, (uint32_t)P[v].nbins, 0u});
+    fills.push_back({(uint32_t *)P[v].dcount, (uint32_t)kDrawCounts, 0u});
     const rhip_clear_states &cs = b.views[v].clear;
     const size_t px = (size_t)P[v].fb_w * P[v].fb_h * P[v].samples;
     if (cs.color_flag && P[v].color) fills.push_back({P[v].color, (uint32_t)px, clearColorWord(cs)});
@@ -230,8 +231,6 @@ int buildBatch(rhip_device d, Batch &b, const rhip_batch_config &c) {
     kb_setup<<<(unsigned)n_tri, 256, 0, s>>>(Pv, T + o_tri);
     kb_clip<<<(unsigned)n_tri, 256, 0, s>>>(Pv, T + o_tri);
   }
-  kb_scan_fans<<<nv, 1024, 0, s>>>(Pv);
-  if (n_tri) kb_clip_fans<<<(unsigned)n_tri, 256, 0, s>>>(Pv, T + o_tri);
   kb_bin_scan<<<nv, 1024, 0, s>>>(Pv);
   if (n_tri) kb_bin_emit<<<(unsigned)n_tri, 256, 0, s>>>(Pv, T + o_tri);
   if (b.samples == 4) {

@@ -22,8 +22,6 @@ constexpr int kCounterSlots = 64, kCounterStride = 16;
 constexpr int kVaryStride = 32;   /* varying slots of a vertex shader output (the reference layout) */
 constexpr int kMaxClipVerts = 12; /* new vertices one clipped triangle can create */
 constexpr int kMaxPoly = 9;       /* polygon vertices after six planes */
-/* 64-block chunks of a draw's 256-triangle blocks, whose fan counts are summed together */
-__host__ __device__ inline int fanChunks(int nblk) { return (nblk + 63) >> 6; }
 constexpr int kMaxFans = kMaxPoly - 3; /* extra triangles one clipped triangle can append */
 /* Binning: a primitive whose quads touch at most kBinFine tiles is listed in
  * each of those tiles; a larger one in each kCoarse x kCoarse-tile coarse bin
@@ -135,6 +133,8 @@ constexpr int kErrClip = 0; /* a clipped polygon exceeded kMaxPoly vertices: the
 constexpr int kErrSlots = 4;
 
 /* PrimSetup.flags */
+/* a draw's device scalars (DrawParams::dcount): all fan triangles past the first of each polygon; triangles to clip */
+constexpr int kCountFans = 0, kCountClip = 9, kDrawCounts = 16;
 constexpr int kPrimLive = 1, kPrimFront = 2, kPrimCoarse = 4, kPrimGlobal = 8;
 
 struct DrawParams {
@@ -163,7 +163,6 @@ struct DrawParams {
   int tiles_x, tiles_y;
   /* geometry */
   const float *verts;
-  const float *clip_raw;
   int stride_f; /* floats per vertex */
   int nverts;
   const int *idx;
@@ -174,15 +173,11 @@ struct DrawParams {
   int *mask;
   float *vary;
   /* clipping: triangle t owns new-vertex slots nverts + t * kMaxClipVerts ... */
-  int *clip_poly; /* kMaxPoly vertex ids + count per triangle of a block that clips */
-  int *fan_first; /* per clipped triangle: id of its second fan triangle (the first keeps its id) */
-  int *blk_clip;  /* per 256-triangle block: triangles that need clipping */
-  int *blk_fans;  /* per block: fan triangles its clipped triangles append */
-  int *blk_fan_off; /* per block: its fans' offset (batched views) */
-  int *chunk_fans;  /* per 64 blocks: their fan triangles (a single draw) */
+  int *clip_poly; /* kMaxPoly vertex ids + count per clipped triangle */
+  int *clip_list; /* the triangles to clip, in no order; their number in dcount */
   int nblk;
-  int *dcount; /* device scalars: [0] appended fan triangles, [1] primitive count, [2] queued fragments,
-                [3] listed fragments, [7] tiles left to the ordered raster, [8] tiles with listed fragments */
+  int *dcount; /* device scalars (kCount...): queued fragments [2], listed fragments [3], tiles left to the
+                  ordered raster [7], tiles with listed fragments [8] */
   /* primitives */
   PrimSetup *prims;
   /* bins: ntiles fine bins of tile x tile pixels, then coarse_x * coarse_y coarse bins of
