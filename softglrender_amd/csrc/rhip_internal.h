@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "rhip_gptr.h"
 #include "rhip_libm.h"
 #include "rhip_stream.h"
 
@@ -46,8 +47,8 @@ struct TexLevel {
 
 /* Device-resident texture descriptor (read with scalar loads by the kernels). */
 struct TexDesc {
-  uint8_t *base;
-  uint8_t *resolved; /* single-sample image of a multisampled colour target */
+  GPtr<uint8_t> base;
+  GPtr<uint8_t> resolved; /* single-sample image of a multisampled colour target */
   int type, format, width, height;
   int layers, levels, layout, msaa;
   int filter_min, filter_mag, wrap, border;
@@ -139,15 +140,15 @@ constexpr int kPrimLive = 1, kPrimFront = 2, kPrimCoarse = 4, kPrimGlobal = 8;
 
 struct DrawParams {
   Uniforms u;
-  const TexDesc *tex[RHS_SLOT_COUNT];
+  GPtr<const TexDesc> tex[RHS_SLOT_COUNT];
   RhsStates st;
   int shading;
   uint32_t defines;
   int need_deriv; /* a sampler of the draw needs dFdx/dFdy (mipmapped minification) */
-  const float *gamma_lut; /* [0, 256): powf(k / 255, 2.2); [256, 512): the PBR output-byte thresholds
+  GPtr<const float> gamma_lut; /* [0, 256): powf(k / 255, 2.2); [256, 512): the PBR output-byte thresholds
                              (host libm, rhip_libm.hip) */
-  const LibmTables *libm; /* the host libm's log2f / exp2f / powf on the device (rhip_libm.h) */
-  const IblTables *ibl;   /* sin / cos tables of the IBL shaders */
+  GPtr<const LibmTables> libm; /* the host libm's log2f / exp2f / powf on the device (rhip_libm.h) */
+  GPtr<const IblTables> ibl;   /* sin / cos tables of the IBL shaders */
   float base_lin[3];      /* powf(base colour, 2.2) by the host libm (PbrSoft.h:235) */
   uint32_t vary_groups; /* stored groups of 4 varying slots (varyGroups) */
   int vary_stride;      /* floats per vertex in `vary`: 4 per stored group */
@@ -155,57 +156,57 @@ struct DrawParams {
   float vp_w, vp_h, o_x, o_y, p_x, p_y;
   float pl_point_size; /* gl->PointSize after the vertex shader: u_pointSize for the base colour shader, else 1 */
   /* framebuffer */
-  uint32_t *color;          /* RGBA8, `samples` per pixel */
-  uint32_t *color_resolved; /* RGBA8 single sample, when samples == 4 */
-  float *depth;             /* f32, `samples` per pixel */
+  GPtr<uint32_t> color;          /* RGBA8, `samples` per pixel */
+  GPtr<uint32_t> color_resolved; /* RGBA8 single sample, when samples == 4 */
+  GPtr<float> depth;             /* f32, `samples` per pixel */
   int fb_w, fb_h;           /* attachment size */
   int samples;              /* 1 or 4 */
   int tiles_x, tiles_y;
   /* geometry */
-  const float *verts;
+  GPtr<const float> verts;
   int stride_f; /* floats per vertex */
   int nverts;
-  const int *idx;
+  GPtr<const int> idx;
   int ntris;
   /* vertex stage outputs */
-  float4 *clip;
-  float4 *frag;
-  int *mask;
-  float *vary;
+  GPtr<float4> clip;
+  GPtr<float4> frag;
+  GPtr<int> mask;
+  GPtr<float> vary;
   /* clipping: triangle t owns new-vertex slots nverts + t * kMaxClipVerts ... */
-  int *clip_poly; /* kMaxPoly vertex ids + count per clipped triangle */
-  int *clip_list; /* the triangles to clip, in no order; their number in dcount */
+  GPtr<int> clip_poly; /* kMaxPoly vertex ids + count per clipped triangle */
+  GPtr<int> clip_list; /* the triangles to clip, in no order; their number in dcount */
   int nblk;
-  int *dcount; /* device scalars (kCount...): queued fragments [2], listed fragments [3], tiles left to the
+  GPtr<int> dcount; /* device scalars (kCount...): queued fragments [2], listed fragments [3], tiles left to the
                   ordered raster [7], tiles with listed fragments [8] */
   /* primitives */
-  PrimSetup *prims;
+  GPtr<PrimSetup> prims;
   /* bins: ntiles fine bins of tile x tile pixels, then coarse_x * coarse_y coarse bins of
    * coarse_tiles x coarse_tiles tiles, then the global bin */
   int tile, coarse_tiles;
   int ntiles, coarse_x, coarse_y, nbins;
-  int *bin_count;  /* [nbins] */
-  int *bin_start;  /* [nbins + 1] */
-  int *bin_cursor; /* [nbins] */
-  int *bin_items;  /* primitive ids, unordered within a bin */
+  GPtr<int> bin_count;  /* [nbins] */
+  GPtr<int> bin_start;  /* [nbins + 1] */
+  GPtr<int> bin_cursor; /* [nbins] */
+  GPtr<int> bin_items;  /* primitive ids, unordered within a bin */
   /* two-phase raster */
-  uint2 *jobs;          /* (pixel | sample mask << 28, winner) per visible fragment; count in dcount[2]
+  GPtr<uint2> jobs;          /* (pixel | sample mask << 28, winner) per visible fragment; count in dcount[2]
                            (the listed ordered raster: dcount[3]) */
-  uint32_t *hiz_bound; /* per coarse bin: depth bound from big triangles covering it */
-  int *hiz_count;      /* per coarse bin: big triangles that bound leaves, -1 if over kHizCap */
-  int *hiz_surv;       /* per coarse bin: those triangles (kHizCap slots) */
-  int *hiz_seed;       /* per coarse bin: nearest clipped polygon covering it, or -1 */
-  int *hiz_poly;       /* per coarse bin: 1 when that polygon's depth range tightened hiz_bound */
+  GPtr<uint32_t> hiz_bound; /* per coarse bin: depth bound from big triangles covering it */
+  GPtr<int> hiz_count;      /* per coarse bin: big triangles that bound leaves, -1 if over kHizCap */
+  GPtr<int> hiz_surv;       /* per coarse bin: those triangles (kHizCap slots) */
+  GPtr<int> hiz_seed;       /* per coarse bin: nearest clipped polygon covering it, or -1 */
+  GPtr<int> hiz_poly;       /* per coarse bin: 1 when that polygon's depth range tightened hiz_bound */
   int hiz_off;         /* 1: no depth-bound culling at all (every triangle is rasterized; for tests) */
   /* listed ordered raster (draws that write no depth): fragments in jobs[0, dcount[3]) */
-  float4 *ord_col;  /* shaded colour per listed fragment */
-  int2 *ord_span;   /* per pixel of a listed tile: its fragments jobs[x, x + y), in API order */
-  int *ord_state;   /* per tile: kOrdEmpty, kOrdListed or kOrdOverflow */
-  int *ord_list;    /* tiles whose fragments did not fit (dcount[7] from the front) and tiles with
+  GPtr<float4> ord_col;  /* shaded colour per listed fragment */
+  GPtr<int2> ord_span;   /* per pixel of a listed tile: its fragments jobs[x, x + y), in API order */
+  GPtr<int> ord_state;   /* per tile: kOrdEmpty, kOrdListed or kOrdOverflow */
+  GPtr<int> ord_list;    /* tiles whose fragments did not fit (dcount[7] from the front) and tiles with
                        listed fragments (dcount[8] from the back) */
   int ord_cap;      /* jobs slots */
-  uint32_t *errors; /* kErrSlots words, see kErrClip */
-  unsigned long long *counters; /* [0] fs invocations, [1] samples written, [2] clip overflows,
+  GPtr<uint32_t> errors; /* kErrSlots words, see kErrClip */
+  GPtr<unsigned long long> counters; /* [0] fs invocations, [1] samples written, [2] clip overflows,
                                    [3] bin items, [4] primitives binned, [5] clipped triangles,
                                    [6] (tile, triangle) pairs skipped by the hierarchical-Z test */
 };

@@ -28,6 +28,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "rhip_gptr.h"
+
 namespace rhip {
 
 enum LibmFn {
@@ -44,8 +46,8 @@ enum LibmFn {
 struct LibmTab {
   uint32_t lo, hi;        /* input bit patterns covered, inclusive (positive floats) */
   double gate;            /* midpoint distance (ulps) at or below which an input may be listed */
-  const uint32_t *bucket; /* ((hi >> 16) - (lo >> 16) + 2) offsets into ent, by input bits >> 16 */
-  const uint32_t *ent;    /* low 16 input bits | 1 << 16 when the host result is one ulp above */
+  GPtr<const uint32_t> bucket; /* ((hi >> 16) - (lo >> 16) + 2) offsets into ent, by input bits >> 16 */
+  GPtr<const uint32_t> ent;    /* low 16 input bits | 1 << 16 when the host result is one ulp above */
 };
 
 struct LibmTables {
