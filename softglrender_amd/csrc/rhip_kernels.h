@@ -2670,117 +2670,198 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
 }
 
 /* The IBL precompute shaders (irradiance: 252 x 63 terms per fragment;
- * prefilter: 1024 samples) on listed fragments. VALU issue bounds it (a term is
- * an importance sample and a cube fetch with correctly rounded divisions), so
- * the ordered sums must not cost as much as the terms: a workgroup takes G
- * fragments and computes 256 / G terms of each at a time; one wavefront (each in
- * turn, while the others go on with the next terms) then adds them in the
- * shader's order from LDS, one lane per fragment and channel, so each sum is the
- * sequential one, bit for bit. G is the most that still leaves 1,024 workgroups
- * (four wavefronts per SIMD): 16 for a face of 128^2, 1 for 32^2 and below. What
- * depends on the draw only is in LDS: the prefilter's half vectors (sample and
- * roughness), the irradiance sum's sines and cosines. With one wavefront per
- * fragment, whose 64 lanes all added every term, the 36 draws of a 512^2 source's
- * maps averaged 763 us; so 243 us, and 147 us with the footprint sampler. */
-constexpr int kIblGroups = 1024, kIblMaxFrags = 16;
+ * prefilter: 1024 samples) on listed fragments. A term is an importance sample
+ * and a cube fetch with correctly rounded divisions, and each fragment's sum is
+ * the sequential one, bit for bit: the terms are many and independent, the sum
+ * is one chain. So a workgroup takes G fragments; eight wavefronts compute up to
+ * two terms a lane each round into LDS, a plane per channel, while a ninth adds
+ * the round before, one lane per fragment and channel, four terms a read. G is
+ * the most that still leaves kIblGroups workgroups, two per CU: 16 for a face of
+ * 128^2, 2 for 32^2. A round's loads and its arithmetic take turns unless other
+ * wavefronts fill in, so two workgroups must fit: nine wavefronts start at the
+ * same SIMD each time, which then holds six, hence at most 80 registers (with 93
+ * and eight of them not spilled, one workgroup ran at a time: 340 us for 250).
+ * What depends on the draw only is in LDS: the prefilter's half vectors (sample
+ * and roughness), the irradiance sum's sines and cosines, the source's
+ * descriptor (two thirds of an irradiance term's vector loads were its level's
+ * offset and size).
+ *
+ * At roughness 0 all half vectors are the normal, so a fragment's 1024 samples
+ * are one sample (sines and cosines times 0 may differ in a zero's sign only,
+ * which no sum below keeps): it is computed once and added 1024 times.
+ *
+ * The maps of a 512^2 source, us a draw: one wavefront per fragment, whose 64
+ * lanes all added every term, 763 on average; terms shared by 256 lanes and
+ * added by each wavefront in turn 143 (irradiance at 32^2 545; prefilter at
+ * 128^2 and roughness 0 164, 64^2 87, 32^2 47, 16^2 45, 8^2 24); so 70 (250; 16,
+ * 100, 35, 23, 15). The 64^2 level is bound by its arithmetic (570 instructions
+ * a sample) and pays for the shared adder; the others gain more. */
+constexpr int kIblGroups = 512, kIblTerms = 512, kIblMaxFrags = 16;
+constexpr int kIblRound = 2 * kIblTerms;                    /* terms of a round: up to two a lane */
+constexpr int kIblPlane = kIblRound + 4 * kIblMaxFrags + 4; /* fragment f's terms start at f (terms of a fragment + 4) */
+
+/* The listed fragment's inputs: its centre sample, else its first inside sample. */
 template <int S>
-__global__ __launch_bounds__(256) void k_ord_shade_ibl(DrawParams P, int need_deriv) {
-  __shared__ float4 terms[2][256 + kIblMaxFrags]; /* fragment f's terms start at f (256 / G + 1): distinct banks */
-  __shared__ float acc[4 * kIblMaxFrags];
+__device__ __forceinline__ Frag iblFrag(const DrawParams &P, uint2 jb, int need_deriv) {
+  const uint32_t pix = jb.x & 0x0fffffffu;
+  const int x = (int)(pix % (uint32_t)P.fb_w), y = (int)(pix / (uint32_t)P.fb_w);
+  const int id = (int)(jb.y >> 2), inst = (int)(jb.y & 3u);
+  const PrimSetup ps = P.prims[id];
+  const Tri T = makeTri(P.frag[ps.v[0]], P.frag[ps.v[1]], P.frag[ps.v[2]]);
+  const float fx = (float)x, fy = (float)y;
+  float4 bs;
+  if (S == 4) {
+    if (!bary(T, fx + 0.5f, fy + 0.5f, bs)) {
+#pragma unroll
+      for (int t = 3; t >= 0; t--) {
+        float4 b;
+        if (bary(T, sampleX(t) + fx, sampleY(t) + fy, b)) bs = b;
+      }
+    }
+  } else {
+    bary(T, fx + 0.5f, fy + 0.5f, bs);
+  }
+  return makeFrag<S, kShadingEnv>(P, ps, T, x, y, bs, inst, need_deriv);
+}
+
+template <int S>
+__global__ __launch_bounds__(kIblTerms + 64) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_ord_shade_ibl(DrawParams P, int need_deriv) {
+  __shared__ float4 planes[2][kIblPlane]; /* [round][channel * kIblPlane + ...] as floats */
+  __shared__ float4 ones[4];              /* the weights' own sum is a sum of weight * 1 */
   __shared__ float hx[1024], hy[1024], hz[1024]; /* half vectors; or sin, cos of phi (hx) and of theta (hy) */
+  __shared__ TexDesc s_tex;
   const int n = min(P.dcount[3], P.ord_cap);
   if (n <= 0) return;
   const bool irradiance = P.shading == RHS_SHADING_IBL_IRRADIANCE;
   int G = 1;
   while (G < kIblMaxFrags && 2 * G * kIblGroups <= n) G *= 2;
   if ((int)blockIdx.x * G >= n) return;
-  const int tpf = 256 / G, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int fi = tid / tpf, ti = tid - fi * tpf;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int total = irradiance ? P.ibl->nphi * P.ibl->ntheta : 1024;
-  const int rounds = (total + tpf - 1) / tpf;
-  const int ntheta = P.ibl->ntheta;
-  const float rtheta = 1.f / (float)ntheta;
+  const TexDesc *src = P.tex[RHS_SLOT_CUBE];
+  const TexDesc *tex = src ? &s_tex : nullptr;
+  if (src)
+    for (int i = tid; i < (int)(sizeof(TexDesc) / 4); i += kIblTerms + 64) ((uint32_t *)&s_tex)[i] = ((const uint32_t *)src)[i];
+  bool same = true;
+  if (tid < 4) ones[tid] = make_float4(1.f, 1.f, 1.f, 1.f);
   if (irradiance) {
-    hx[tid] = P.ibl->sphi[tid], hx[256 + tid] = P.ibl->cphi[tid];
+    same = false;
+    if (tid < 256) hx[tid] = P.ibl->sphi[tid], hx[256 + tid] = P.ibl->cphi[tid];
     if (tid < 64) hy[tid] = P.ibl->stheta[tid], hy[64 + tid] = P.ibl->ctheta[tid];
   } else {
-    for (int i = tid; i < 1024; i += 256) {
+    for (int i = tid; i < 1024; i += kIblTerms + 64) {
       const f3 h = prefHalf(P, i);
       hx[i] = h.x, hy[i] = h.y, hz[i] = h.z;
+      same = same && h.x == 0.f && h.y == 0.f && h.z == 1.f;
     }
   }
+  const int sf = lane >> 2, sc = lane & 3;
+  /* channel sc of fragment j from its sum; every lane of the quad calls it */
+  auto finish = [&](int j, float a) {
+    const float tw = __shfl(a, lane | 3);
+    float v = 1.f;
+    if (sc < 3) v = irradiance ? (a * kPI) * (1.0f / (float)total) : a / tw;
+    ((float *)&P.ord_col[j])[sc] = gclamp(v, 0.f, 1.f);
+  };
+  if (__syncthreads_and(same)) {
+    for (int t = w * (int)gridDim.x + (int)blockIdx.x; t * 16 < n; t += (kIblTerms / 64 + 1) * (int)gridDim.x) {
+      const int j = t * 16 + sf;
+      const uint2 jb = j < n ? P.jobs[j] : make_uint2(kListVoid, 0u);
+      if (jb.x == kListVoid) continue;
+      const PrefSetup pst = prefSetup(P, iblFrag<S>(P, jb, need_deriv));
+      const float4 s = prefSample(P, tex, pst, {0.f, 0.f, 1.f});
+      const float v = sc == 0 ? s.x : sc == 1 ? s.y : sc == 2 ? s.z : 1.f;
+      float a = 0.f;
+#pragma unroll 16
+      for (int i = 0; i < 1024; i++) a = fmaf(v, s.w, a);
+      finish(j, a);
+    }
+    return;
+  }
+
+  const int lpf = kIblTerms / G;                      /* lanes of a fragment */
+  const int tpf = total > 2 * lpf ? 2 * lpf : lpf;    /* terms of a fragment in a round */
+  const int rounds = (total + tpf - 1) / tpf;
+  const bool adder = w == kIblTerms / 64;
+  const int fi = tid / lpf, ti = tid - fi * lpf;
+  const int ntheta = P.ibl->ntheta;
+  const float rtheta = 1.f / (float)ntheta;
+  int parity = 0, pj = -1, pr = 0; /* the round to be added next: its fragments and its number (pj < 0: none) */
+  float a = 0.f;
+  /* the ninth wavefront: adds the terms of round pr of the fragments from pj (lanes past 4 G idle) */
+  auto addRound = [&](int buf) {
+    if (pj < 0 || lane >= 4 * G) return;
+    const float *pl = (const float *)planes[buf] + sf * (tpf + 4);
+    const float4 *v = (const float4 *)(pl + sc * kIblPlane);
+    const float4 *m = sc == 3 ? ones : (const float4 *)(pl + 3 * kIblPlane);
+    if (pr == 0) a = 0.f;
+    float4 cv[4], cm[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) cv[i] = v[i], cm[i] = m[i];
+    for (int q = 4;; q += 4) { /* the next four reads are in flight while these are added */
+      const bool more = q < tpf / 4;
+      float4 nv[4], nm[4];
+      const int at = more ? q : 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) nv[i] = v[at + i], nm[i] = m[(sc == 3 ? 0 : at) + i];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        a = fmaf(cv[i].x, cm[i].x, a);
+        a = fmaf(cv[i].y, cm[i].y, a);
+        a = fmaf(cv[i].z, cm[i].z, a);
+        a = fmaf(cv[i].w, cm[i].w, a);
+      }
+      if (!more) break;
+#pragma unroll
+      for (int i = 0; i < 4; i++) cv[i] = nv[i], cm[i] = nm[i];
+    }
+    if (pr == rounds - 1) {
+      const int j = pj + sf;
+      if (j < n && P.jobs[j].x != kListVoid) finish(j, a);
+    }
+  };
   for (int j0 = blockIdx.x * G; j0 < n; j0 += gridDim.x * G) {
-    const int j = j0 + fi;
-    const uint2 jb = j < n ? P.jobs[j] : make_uint2(kListVoid, 0u);
-    const bool act = jb.x != kListVoid;
+    bool act = false;
     IrrSetup ist{};
     PrefSetup pst{};
-    if (act) {
-      const uint32_t pix = jb.x & 0x0fffffffu;
-      const int x = (int)(pix % (uint32_t)P.fb_w), y = (int)(pix / (uint32_t)P.fb_w);
-      const int id = (int)(jb.y >> 2), inst = (int)(jb.y & 3u);
-      const PrimSetup ps = P.prims[id];
-      const Tri T = makeTri(P.frag[ps.v[0]], P.frag[ps.v[1]], P.frag[ps.v[2]]);
-      const float fx = (float)x, fy = (float)y;
-      float4 bs;
-      if (S == 4) {
-        if (!bary(T, fx + 0.5f, fy + 0.5f, bs)) {
-#pragma unroll
-          for (int t = 3; t >= 0; t--) {
-            float4 b;
-            if (bary(T, sampleX(t) + fx, sampleY(t) + fy, b)) bs = b;
-          }
-        }
-      } else {
-        bary(T, fx + 0.5f, fy + 0.5f, bs);
+    if (!adder) {
+      const int j = j0 + fi;
+      const uint2 jb = j < n ? P.jobs[j] : make_uint2(kListVoid, 0u);
+      act = jb.x != kListVoid;
+      if (act) {
+        const Frag f = iblFrag<S>(P, jb, need_deriv);
+        if (irradiance)
+          ist = irrSetup(f);
+        else
+          pst = prefSetup(P, f);
       }
-      const Frag f = makeFrag<S, kShadingEnv>(P, ps, T, x, y, bs, inst, need_deriv);
-      if (irradiance)
-        ist = irrSetup(f);
-      else
-        pst = prefSetup(P, f);
     }
-    if (tid < 4 * G) acc[tid] = 0.f;
-    __syncthreads(); /* acc and the half vectors; the last group's sums are read */
-    const int sf = lane >> 2, sc = lane & 3;
-    /* adds round r's terms; the wavefront's lanes past 4 G idle */
-    auto addRound = [&](int r) {
-      if (lane >= 4 * G) return;
-      const float *t = (const float *)(terms[r & 1] + sf * (tpf + 1));
-      float a = acc[lane];
-#pragma unroll 8
-      for (int q = 0; q < tpf; q++) {
-        const float v = t[4 * q + sc], wgt = t[4 * q + 3];
-        a = fmaf(v, sc == 3 ? 1.f : wgt, a); /* channel 3: the weights' own sum */
-      }
-      acc[lane] = a;
-    };
     for (int r = 0; r < rounds; r++) {
-      const int k = r * tpf + ti;
-      float4 t = make_float4(0.f, 0.f, 0.f, 0.f); /* adds nothing to a sum that is not negative */
-      if (act && k < total) {
-        if (irradiance) {
-          /* k / ntheta: k + 0.5 is at least 0.5 / ntheta from a multiple, far beyond the product's rounding */
-          const int i = (int)(((float)k + 0.5f) * rtheta), m = k - i * ntheta;
-          t = irrTerm(P, ist, hx[i], hx[256 + i], hy[m], hy[64 + m]);
-        } else {
-          t = prefSample(P, pst, {hx[k], hy[k], hz[k]});
+      if (adder) {
+        addRound(parity ^ 1);
+        pj = j0, pr = r;
+      } else {
+        for (int q = ti; q < tpf; q += lpf) {
+          const int k = r * tpf + q;
+          float4 t = make_float4(0.f, 0.f, 0.f, 0.f); /* adds nothing to a sum that is not negative */
+          if (act && k < total) {
+            if (irradiance) {
+              /* k / ntheta: k + 0.5 is at least 0.5 / ntheta from a multiple, far beyond the product's rounding */
+              const int i = (int)(((float)k + 0.5f) * rtheta), m = k - i * ntheta;
+              t = irrTerm(tex, ist, hx[i], hx[256 + i], hy[m], hy[64 + m]);
+            } else {
+              t = prefSample(P, tex, pst, {hx[k], hy[k], hz[k]});
+            }
+          }
+          float *pl = (float *)planes[parity] + fi * (tpf + 4) + q;
+          pl[0] = t.x, pl[kIblPlane] = t.y, pl[2 * kIblPlane] = t.z, pl[3 * kIblPlane] = t.w;
         }
       }
-      terms[r & 1][fi * (tpf + 1) + ti] = t;
-      __syncthreads();
-      if (w == (r & 3)) addRound(r);
+      parity ^= 1;
+      __syncthreads(); /* this round's terms are written, and the last round's are read */
     }
-    __syncthreads();
-    if (act && ti == 0) {
-      const f3 a{acc[4 * fi], acc[4 * fi + 1], acc[4 * fi + 2]};
-      const float tw = acc[4 * fi + 3];
-      const RGBAf c = irradiance ? irrFinish(a, (float)total) : RGBAf{a.x / tw, a.y / tw, a.z / tw, 1.f};
-      P.ord_col[j] = make_float4(gclamp(c.r, 0.f, 1.f), gclamp(c.g, 0.f, 1.f), gclamp(c.b, 0.f, 1.f),
-                                 gclamp(c.a, 0.f, 1.f));
-    }
-    __syncthreads(); /* the sums are read before the next group clears them */
   }
+  if (adder) addRound(parity ^ 1);
 }
 
 /* Each pixel's listed fragments written to its samples in order, blended when

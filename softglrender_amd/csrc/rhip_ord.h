@@ -22,7 +22,7 @@ void launchOrdShade(const DrawParams &P, int grid, int need_deriv, hipStream_t s
     case RHS_SHADING_IBL_IRRADIANCE:
     case RHS_SHADING_IBL_PREFILTER:
       /* a workgroup takes 1 to 16 fragments; `grid` blocks of 256 lanes cover them one lane each */
-      RHIP_LAUNCH(k_ord_shade_ibl<S>, std::min(grid * 256, 2 * kIblGroups), 256, st, P, need_deriv);
+      RHIP_LAUNCH(k_ord_shade_ibl<S>, std::min(grid * 256, 2 * kIblGroups), kIblTerms + 64, st, P, need_deriv);
       break;
     case RHS_SHADING_SKYBOX:
     case RHS_SHADING_FXAA: RHIP_LAUNCH(k_ord_shade<S RHIP_COMMA kShadingEnv>, grid, 256, st, P, need_deriv); break;

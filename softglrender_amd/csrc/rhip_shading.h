@@ -930,12 +930,12 @@ __device__ __forceinline__ IrrSetup irrSetup(const Frag &f) {
  * colour times cos(theta), and sin(theta). The reference build fuses the last
  * product into the running sum (irrAdd), and the sample vector into two
  * multiply-adds. */
-__device__ __forceinline__ float4 irrTerm(const DrawParams &P, const IrrSetup &s, float sp, float cp, float st, float ct) {
+__device__ __forceinline__ float4 irrTerm(const TexDesc *tex, const IrrSetup &s, float sp, float cp, float st, float ct) {
   const f3 ts{st * cp, st * sp, ct};
   const f3 sv{fmaf(s.N.x, ts.z, fmaf(s.up.x, ts.y, s.right.x * ts.x)),
               fmaf(s.N.y, ts.z, fmaf(s.up.y, ts.y, s.right.y * ts.x)),
               fmaf(s.N.z, ts.z, fmaf(s.up.z, ts.y, s.right.z * ts.x))};
-  const RGBAf c = texCube(P.tex[RHS_SLOT_CUBE], sv, 0.f);
+  const RGBAf c = texCube(tex, sv, 0.f);
   return make_float4(c.r * ct, c.g * ct, c.b * ct, st);
 }
 __device__ __forceinline__ f3 irrAdd(f3 irr, float4 t) {
@@ -952,7 +952,7 @@ __device__ RGBAf fsIrradiance(const DrawParams &P, const Frag &f) {
   float nr = 0.f;
   for (int i = 0; i < T.nphi; i++)
     for (int j = 0; j < T.ntheta; j++) {
-      irr = irrAdd(irr, irrTerm(P, s, T.sphi[i], T.cphi[i], T.stheta[j], T.ctheta[j]));
+      irr = irrAdd(irr, irrTerm(P.tex[RHS_SLOT_CUBE], s, T.sphi[i], T.cphi[i], T.stheta[j], T.ctheta[j]));
       nr += 1.f;
     }
   return irrFinish(irr, nr);
@@ -992,7 +992,7 @@ __device__ __forceinline__ f3 prefHalf(const DrawParams &P, uint32_t i) {
   return {T.hcos[i] * sinT, T.hsin[i] * sinT, cosT};
 }
 /* The sample of half vector Ht: the source texel's colour and N.L (the sample counts only when N.L > 0). */
-__device__ __forceinline__ float4 prefSample(const DrawParams &P, const PrefSetup &s, f3 Ht) {
+__device__ __forceinline__ float4 prefSample(const DrawParams &P, const TexDesc *tex, const PrefSetup &s, f3 Ht) {
   const f3 N = s.N, V = s.V, tangent = s.tangent, bitangent = s.bitangent;
   const float ra2 = s.ra2;
   const f3 H = nrm3b({fmaf(N.x, Ht.z, fmaf(bitangent.x, Ht.y, tangent.x * Ht.x)),
@@ -1008,7 +1008,7 @@ __device__ __forceinline__ float4 prefSample(const DrawParams &P, const PrefSetu
   const float pdf = D * NdotH / (4.0f * HdotV) + 0.0001f;
   const float saSample = 1.0f / fmaf(1024.0f, pdf, 0.0001f);
   const float mip = s.rough == 0.0f ? 0.0f : 0.5f * hlog2f(P.libm, saSample / s.saTexel);
-  const RGBAf c = texCube(P.tex[RHS_SLOT_CUBE], L, mip);
+  const RGBAf c = texCube(tex, L, mip);
   return make_float4(c.r, c.g, c.b, NdotL);
 }
 __device__ RGBAf fsPrefilter(const DrawParams &P, const Frag &f) {
@@ -1016,7 +1016,7 @@ __device__ RGBAf fsPrefilter(const DrawParams &P, const Frag &f) {
   f3 acc{0.f, 0.f, 0.f};
   float tw = 0.f;
   for (uint32_t i = 0; i < 1024u; i++) {
-    const float4 t = prefSample(P, s, prefHalf(P, i));
+    const float4 t = prefSample(P, P.tex[RHS_SLOT_CUBE], s, prefHalf(P, i));
     if (t.w > 0.0f) {
       acc = {fmaf(t.x, t.w, acc.x), fmaf(t.y, t.w, acc.y), fmaf(t.z, t.w, acc.z)};
       tw += t.w;

@@ -89,3 +89,36 @@ def test_ibl_groups_match_checker(renderer, size):
         st.end()
         st.read(tex)
     _check(renderer, scenes.Scene(f"ibl face {size}", st, size, size, False))
+
+
+@pytest.mark.parametrize("size", [1, 5, 40])
+def test_ibl_one_direction_matches_checker(renderer, size):
+    """Roughness 0, where a fragment's samples all have one direction (16 fragments to a wavefront, the last not full),
+    next to the least roughness that spreads them; and an irradiance face of 2 fragments to a workgroup."""
+    st = S.Stream()
+    v, idx = scenes.cube_mesh()
+    st.vao(1, v, idx)
+    st.texture(10, 16, 16, type=S.TEX_CUBE, mipmaps=True, usage=S.USAGE_SAMPLER | S.USAGE_UPLOAD,
+               filter_min=S.FILTER_LINEAR_MIPMAP_LINEAR, filter_mag=S.FILTER_LINEAR, wrap=S.WRAP_CLAMP_TO_EDGE)
+    st.tex_data(10, scenes.env_cube_faces(16, 5))
+    st.frame()
+    proj = scenes.projection(math.radians(90.0), 1.0, 0.1)
+    jobs = [(11 + k, size, S.SHADING_IBL_PREFILTER, struct.pack("<2f", 16.0, rough) + bytes(40))
+            for k, rough in enumerate((0.0, 1e-12, 0.02))]
+    if size == 40:
+        jobs.append((14, 33, S.SHADING_IBL_IRRADIANCE, bytes(48)))
+    for face, (tex, n, shading, mat) in enumerate(jobs):
+        center, up = scenes._CUBE_VIEWS[face]
+        turn = np.eye(4)
+        turn[:3, :3] = scenes.look_at((0, 0, 0), center, up)[:3, :3]
+        print(f"[gpu] face of {n}^2, shader {shading}", flush=True)
+        st.texture(tex, n, n, usage=S.USAGE_COLOR)
+        st.tex_init(tex)
+        st.fbo(tex, color=tex)
+        st.begin(tex, True, False, (0, 0, 0, 0), 1.0)
+        st.viewport(0, 0, n, n)
+        st.draw(1, shading, 0, S.RenderStates(), S.uniforms_model(np.eye(4), proj @ turn), bytes(64), mat,
+                samplers=[(S.SLOT_CUBE, 10)])
+        st.end()
+        st.read(tex)
+    _check(renderer, scenes.Scene(f"ibl one direction {size}", st, size, size, False))
