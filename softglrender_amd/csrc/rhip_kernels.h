@@ -2259,12 +2259,80 @@ constexpr uint32_t kListVoid = 0xffffffffu; /* a jobs slot reserved by a tile th
 
 constexpr int kListStage = 96; /* triangles of a window whose walk data is staged in LDS */
 
-/* One tile by one workgroup, one wavefront per 8x8 quarter. A wavefront takes
- * the window's triangles 64 at a time and spreads their (triangle, pixel) pairs
- * over its lanes, 64 pairs per round; fragments are listed in round and lane
- * order, which is primitive-id order for every pixel. */
+/* The exact test of pixel (x, y) against a triangle: the fragments it gives, one
+ * for each quad of the triangle that has it (bit iy * 2 + ix; none: 0), and the
+ * samples they write. Coverage, z and the depth clip (RendererSoft.cpp:776-799),
+ * then the depth test against the samples' depths `dp`, which nothing in this
+ * draw can change. */
 template <int S>
-__device__ __forceinline__ void listTile(const DrawParams &P, int tile) {
+__device__ __forceinline__ uint32_t pairQuads(const DrawParams &P, const Tri &T, float mnx, float mxx, float mny, float mxy,
+                                              int bcx, int bcy, int x, int y, const float *dp, uint32_t &smask) {
+  smask = 1u;
+  int qa, qb;
+  const int nqx = axisQuads(mnx, mxx, bcx, x, qa, qb);
+  const int nqy = nqx ? axisQuads(mny, mxy, bcy, y, qa, qb) : 0;
+  if (!nqx || !nqy) return 0u;
+  const float fx = (float)x, fy = (float)y;
+  const bool hasD = P.depth != nullptr;
+  const int dfunc = P.st.depthFunc;
+  bool sin[4];
+  float sz[4];
+  bool pin;
+  if (S == 4) {
+    pin = false;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      float4 bc;
+      sin[s] = bary(T, sampleX(s) + fx, sampleY(s) + fy, bc);
+      sz[s] = 0.f;
+      pin = pin || sin[s];
+      if (!sin[s]) continue;
+      sz[s] = dpps3(bc, T.z);
+      if (sz[s] < 0.f || sz[s] > 1.f) sin[s] = false;
+    }
+  } else {
+    float4 bc;
+    sin[0] = bary(T, fx + 0.5f, fy + 0.5f, bc);
+    pin = sin[0];
+    sz[0] = pin ? dpps3(bc, T.z) : 0.f;
+  }
+  if (pin && P.st.depthTest) {
+    if (S == 4) {
+      bool any = false;
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        if (!sin[s]) continue;
+        if (hasD) sin[s] = depthPass(gclamp(sz[s], 0.f, 1.f), dp[s], dfunc);
+        any = any || sin[s];
+      }
+      pin = any;
+    } else {
+      pin = hasD ? depthPass(gclamp(sz[0], 0.f, 1.f), dp[0], dfunc) : true;
+    }
+  }
+  if (!pin) return 0u;
+  if (S == 4) {
+    smask = 0;
+#pragma unroll
+    for (int s = 0; s < 4; s++) smask |= (sin[s] ? 1u : 0u) << s;
+  }
+  const uint32_t row = nqx == 2 ? 3u : 1u;
+  return nqy == 2 ? row | row << 2 : row;
+}
+
+/* One tile by one workgroup, one wavefront per 8x8 quarter. With more than
+ * kListDirect bin entries a wavefront takes the window's triangles 64 at a time
+ * and spreads their (triangle, pixel) pairs over its lanes, 64 pairs per round;
+ * fragments are listed in round and lane order, which is primitive-id order for
+ * every pixel. With fewer (a full-screen pass, a cube face) a lane keeps its
+ * pixel and tests the triangles one after another: no pairs, queues or ranks,
+ * only the triangles in LDS. The skybox and the FXAA quad of a 1366 x 768 frame
+ * took 142 us each to list (now 88: a tile's chain of loads, bin to triangle to
+ * vertex, at three workgroups per CU). Its tiles join the list of tiles with
+ * fragments one atomic per workgroup. True if the tile has any. */
+constexpr int kListDirect = 8; /* a byte of quads and samples each in a lane's 64 bits */
+template <int S>
+__device__ __forceinline__ bool listTile(const DrawParams &P, int tile) {
   __shared__ uint32_t win[kOrdWin];
   __shared__ float4 s_stage[kListStage][5];
   __shared__ uint2 s_frag[4][kListCap];
@@ -2291,7 +2359,7 @@ __device__ __forceinline__ void listTile(const DrawParams &P, int tile) {
   const int n = tb.total();
   if (n == 0) {
     if (lp == 0) P.ord_state[tile] = kOrdEmpty;
-    return;
+    return false;
   }
   const float lx[4] = {0.375f, 0.875f, 0.125f, 0.625f};
   const float ly[4] = {0.875f, 0.625f, 0.375f, 0.125f};
@@ -2329,8 +2397,65 @@ __device__ __forceinline__ void listTile(const DrawParams &P, int tile) {
   unsigned long long nculled = 0;
   int wn = 0;        /* fragments this wavefront has listed */
   bool full = false; /* its list overflowed (wave-uniform) */
+  auto stage = [&](int i, int id) {
+    const PrimSetup ps = P.prims[id];
+    const Tri T = makeTri(P.frag[ps.v[0]], P.frag[ps.v[1]], P.frag[ps.v[2]]);
+    s_stage[i][0] = make_float4(__int_as_float(ps.qx0), __int_as_float(ps.qx1), __int_as_float(ps.qy0),
+                                __int_as_float(ps.qy1));
+    s_stage[i][1] = make_float4(ps.min_x, ps.max_x, ps.min_y, ps.max_y);
+    s_stage[i][2] = make_float4(__int_as_float(ps.bcx), __int_as_float(ps.bcy), T.v0x, T.v0y);
+    s_stage[i][3] = make_float4(T.a0, T.a1, T.b0, T.b1);
+    s_stage[i][4] = make_float4(T.uz, T.z[0], T.z[1], T.z[2]);
+  };
+  /* bin entry i has to be walked in this tile */
+  auto wanted = [&](int i, int id) {
+    const PrimSetup &ps = P.prims[id];
+    if (i >= tb.n[0] && (ps.qx0 > X1 || ps.qx1 < tx0 || ps.qy0 > Y1 || ps.qy1 < ty0)) return false;
+    if (!(hiz && zCulled(ps, bound, mx))) return true;
+    nculled++;
+    return false;
+  };
+  const bool direct = n <= kListDirect;
+  int dm = 0;                    /* the direct walk: its triangles, in primitive order in win and s_stage */
+  unsigned long long dcov = 0;   /* quads | samples << 4 of each */
+  if (direct) {
+    const int id = lp < n ? tb.at(P, lp) : 0;
+    const bool keep = lp < n && id <= maxid && wanted(lp, id);
+    const unsigned long long kb = __ballot(keep); /* of the first wavefront, which has them all */
+    if (wave == 0) {
+      int rank = 0;
+      for (int i = 0; i < n; i++) rank += (((kb >> i) & 1ull) && __builtin_amdgcn_readlane(id, i) < id) ? 1 : 0;
+      if (keep) {
+        win[rank] = (uint32_t)id;
+        stage(rank, id);
+      }
+      if (lane == 0) s_n = __popcll(kb);
+    }
+    __syncthreads();
+    dm = s_n;
+    int c = 0;
+    if (inFb) {
+      for (int k = 0; k < dm; k++) {
+        const float4 d0 = s_stage[k][0], d1 = s_stage[k][1], d2 = s_stage[k][2], d3 = s_stage[k][3], d4 = s_stage[k][4];
+        if (px < __float_as_int(d0.x) || px > __float_as_int(d0.y) || py < __float_as_int(d0.z) ||
+            py > __float_as_int(d0.w))
+          continue;
+        Tri T;
+        T.v0x = d2.z, T.v0y = d2.w, T.a0 = d3.x, T.a1 = d3.y, T.b0 = d3.z, T.b1 = d3.w;
+        T.uz = d4.x, T.z[0] = d4.y, T.z[1] = d4.z, T.z[2] = d4.w;
+        if (pixelSurelyOut<S>(T, px, py)) continue;
+        uint32_t smask;
+        const uint32_t qm = pairQuads<S>(P, T, d1.x, d1.y, d1.z, d1.w, __float_as_int(d2.x), __float_as_int(d2.y), px, py,
+                                         dep, smask);
+        if (qm) dcov |= (unsigned long long)(qm | smask << 4) << (8 * k);
+        c += __popc(qm);
+      }
+    }
+    s_cnt[pl] = c;
+    __syncthreads();
+  }
   int lo = 0;
-  while (lo <= maxid) {
+  while (!direct && lo <= maxid) {
     int hi = maxid;
     if (n > kOrdWin) {
       /* the largest hi with at most kOrdWin entries in [lo, hi] */
@@ -2357,29 +2482,13 @@ __device__ __forceinline__ void listTile(const DrawParams &P, int tile) {
     }
     for (int i = lp; i < n; i += 256) {
       const int id = tb.at(P, i);
-      if (id < lo || id > hi) continue;
-      const PrimSetup &ps = P.prims[id];
-      if (i >= tb.n[0] && (ps.qx0 > X1 || ps.qx1 < tx0 || ps.qy0 > Y1 || ps.qy1 < ty0)) continue;
-      if (hiz && zCulled(ps, bound, mx)) {
-        nculled++;
-        continue;
-      }
-      win[atomicAdd(&s_n, 1)] = (uint32_t)id;
+      if (id >= lo && id <= hi && wanted(i, id)) win[atomicAdd(&s_n, 1)] = (uint32_t)id;
     }
     __syncthreads();
     const int m = s_n;
     sortIds(win, m);
     const int ms = min(m, kListStage);
-    for (int i = lp; i < ms; i += 256) {
-      const PrimSetup ps = P.prims[win[i]];
-      const Tri T = makeTri(P.frag[ps.v[0]], P.frag[ps.v[1]], P.frag[ps.v[2]]);
-      s_stage[i][0] = make_float4(__int_as_float(ps.qx0), __int_as_float(ps.qx1), __int_as_float(ps.qy0),
-                                  __int_as_float(ps.qy1));
-      s_stage[i][1] = make_float4(ps.min_x, ps.max_x, ps.min_y, ps.max_y);
-      s_stage[i][2] = make_float4(__int_as_float(ps.bcx), __int_as_float(ps.bcy), T.v0x, T.v0y);
-      s_stage[i][3] = make_float4(T.a0, T.a1, T.b0, T.b1);
-      s_stage[i][4] = make_float4(T.uz, T.z[0], T.z[1], T.z[2]);
-    }
+    for (int i = lp; i < ms; i += 256) stage(i, (int)win[i]);
     __syncthreads();
 
     for (int c0 = 0; c0 < m && !full; c0 += 64) {
@@ -2433,62 +2542,10 @@ __device__ __forceinline__ void listTile(const DrawParams &P, int tile) {
             bcx = ps.bcx, bcy = ps.bcy;
             T = makeTri(P.frag[ps.v[0]], P.frag[ps.v[1]], P.frag[ps.v[2]]);
           }
-          int qa, qb;
-          const int nqx = axisQuads(mnx, mxx, bcx, x, qa, qb);
-          const int nqy = nqx ? axisQuads(mny, mxy, bcy, y, qa, qb) : 0;
-          if (nqx && nqy) {
-            const float fx = (float)x, fy = (float)y;
-            const float *dp = &s_dep[((y - ty0) * kTile + (x - tx0)) * S];
-            /* coverage, z and the depth clip (RendererSoft.cpp:776-799), then
-             * the depth test, which nothing in this draw can change */
-            bool sin[4];
-            float sz[4];
-            bool pin;
-            if (S == 4) {
-              pin = false;
-#pragma unroll
-              for (int s = 0; s < 4; s++) {
-                float4 bc;
-                sin[s] = bary(T, lx[s] + fx, ly[s] + fy, bc);
-                sz[s] = 0.f;
-                pin = pin || sin[s];
-                if (!sin[s]) continue;
-                sz[s] = dpps3(bc, T.z);
-                if (sz[s] < 0.f || sz[s] > 1.f) sin[s] = false;
-              }
-            } else {
-              float4 bc;
-              sin[0] = bary(T, fx + 0.5f, fy + 0.5f, bc);
-              pin = sin[0];
-              sz[0] = pin ? dpps3(bc, T.z) : 0.f;
-            }
-            if (pin && P.st.depthTest) {
-              if (S == 4) {
-                bool any = false;
-#pragma unroll
-                for (int s = 0; s < 4; s++) {
-                  if (!sin[s]) continue;
-                  if (hasD) sin[s] = depthPass(gclamp(sz[s], 0.f, 1.f), dp[s], dfunc);
-                  any = any || sin[s];
-                }
-                pin = any;
-              } else {
-                pin = hasD ? depthPass(gclamp(sz[0], 0.f, 1.f), dp[0], dfunc) : true;
-              }
-            }
-            if (pin) {
-              uint32_t smask = 1u;
-              if (S == 4) {
-                smask = 0;
-#pragma unroll
-                for (int s = 0; s < 4; s++) smask |= (sin[s] ? 1u : 0u) << s;
-              }
-              for (int iy = 0; iy < nqy; iy++)
-                for (int ix = 0; ix < nqx; ix++) qm |= 1u << (iy * 2 + ix);
-              nI = nqx * nqy;
-              word = (uint32_t)((size_t)y * P.fb_w + x) | (smask << 28);
-            }
-          }
+          uint32_t smask;
+          qm = pairQuads<S>(P, T, mnx, mxx, mny, mxy, bcx, bcy, x, y, &s_dep[((y - ty0) * kTile + (x - tx0)) * S], smask);
+          nI = __popc(qm);
+          word = (uint32_t)((size_t)y * P.fb_w + x) | (smask << 28);
         }
         const int pos = waveInclusiveScan(nI);
         const int tot = __builtin_amdgcn_readlane(pos, 63);
@@ -2589,7 +2646,7 @@ __device__ __forceinline__ void listTile(const DrawParams &P, int tile) {
       P.ord_state[tile] = kOrdOverflow;
       P.ord_list[atomicAdd(&P.dcount[7], 1)] = tile;
     }
-    return;
+    return false;
   }
   int base = gb + inc - c;
   for (int v = 0; v < wave; v++) base += s_wn[v];
@@ -2599,12 +2656,16 @@ __device__ __forceinline__ void listTile(const DrawParams &P, int tile) {
     const uint32_t rk = s_rank[wave][e];
     P.jobs[s_cnt[rk & 255u] + (int)(rk >> 8)] = s_frag[wave][e];
   }
-  if (inFb) P.ord_span[pix] = make_int2(base, c);
-  if (lp == 0) {
-    P.ord_state[tile] = kOrdListed;
-    if (all) P.ord_list[P.ntiles - 1 - atomicAdd(&P.dcount[8], 1)] = tile;
+  int at = base;
+  for (int k = 0; k < dm; k++) {
+    const uint32_t v = (uint32_t)(dcov >> (8 * k)) & 255u;
+    for (int f = 0; f < 4; f++)
+      if ((v >> f) & 1u) P.jobs[at++] = make_uint2((uint32_t)pix | (v >> 4) << 28, (win[k] << 2) | (uint32_t)f);
   }
+  if (inFb) P.ord_span[pix] = make_int2(base, c);
+  if (lp == 0) P.ord_state[tile] = kOrdListed;
   waveAddCounter(P, 6, nculled);
+  return all > 0;
 }
 
 /* Tiles dealt round-robin to a grid that fits the GPU at once: most tiles of a
@@ -2629,10 +2690,20 @@ __global__ __launch_bounds__(256) void k_ord_list(DrawParams P) {
     }
     __syncthreads();
     const int nt = s_nt;
+    int nl = 0; /* tiles with listed fragments take the places of those already walked, and the list in one go */
     for (int i = 0; i < nt; i++) {
-      listTile<S>(P, s_tiles[i]);
+      const int tile = s_tiles[i];
+      const bool listed = listTile<S>(P, tile);
       __syncthreads();
+      if (listed) {
+        if (threadIdx.x == 0) s_tiles[nl] = tile;
+        nl++;
+      }
     }
+    if (threadIdx.x == 0 && nl) s_nt = atomicAdd(&P.dcount[8], nl);
+    __syncthreads();
+    if ((int)threadIdx.x < nl) P.ord_list[P.ntiles - 1 - s_nt - (int)threadIdx.x] = s_tiles[threadIdx.x];
+    __syncthreads();
   }
 }
 
