@@ -35,14 +35,16 @@ constexpr int kNnUpdateBlocks = (kNnParams + 15) / 16; /* k_nn_update: 16 parame
 
 /* bf16 operands packed for MFMA (device): W1 with b1 in column 24, W2, W3
  * padded to 16 rows, and the transposes backward needs; biases of layers 2, 3.
- * w2r, w3r and w2tr are W2, W3 and W2^T with their columns in the order
- * nnRegUnit gives, for kernels that keep activations in registers. */
+ * w2r and w3r are W2 and W3 with their columns in the order nnRegUnit gives, for
+ * inference, which takes its operands from result tiles as they are. */
 struct NnPacked {
   __bf16 w1[kNnHid * kNnK1];
+  __bf16 w2[kNnHid * kNnHid];
+  __bf16 w3[16 * kNnHid];
+  __bf16 w2t[kNnHid * kNnHid];
   __bf16 w3t[kNnHid * 32];
   __bf16 w2r[kNnHid * kNnHid];
   __bf16 w3r[16 * kNnHid];
-  __bf16 w2tr[kNnHid * kNnHid];
   float b2[kNnHid];
   float b3[16];
 };
@@ -697,6 +699,28 @@ __device__ __forceinline__ bf16x8 reluPackNan(f32x4 lo, f32x4 hi) {
   return o;
 }
 
+/* The B operand of a layer in the units' own order from two result tiles packed
+ * as reluPackNan does: lane (g, c) wants units 8g .. 8g+7 of the 32, which are in
+ * lanes (2 (g & 1), c) and (2 (g & 1) + 1, c) of tile g >> 1. With the tiles' rows
+ * of 16 lanes as [0 1 2 3], exchanging the first tile's upper half with the
+ * second's lower one gives [a0 a1 b0 b1] and [a2 a3 b2 b3], and exchanging odd
+ * rows with even ones then [a0 a2 b0 b2] and [a1 a3 b1 b3]. Training keeps this
+ * order: a product's sum over K depends on it in the last bit, and 64 steps of
+ * Adam make that 1e-5 in the weights. */
+__device__ __forceinline__ bf16x8 unitOrder(bf16x8 t) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const u32x4 x = __builtin_bit_cast(u32x4, t);
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const u32x2 h = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(x[i], x[2 + i], false, false));
+    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(h[0], h[1], false, false));
+    o[i] = r[0], o[2 + i] = r[1];
+  }
+  return __builtin_bit_cast(bf16x8, o);
+}
+
 /* sum over the 16 rows of a product tile: MFMA with an all-ones operand */
 __device__ __forceinline__ bf16x8 onesOp() {
   bf16x8 o;
@@ -709,8 +733,8 @@ __device__ __forceinline__ bf16x8 onesOp() {
  * drawn from [first, first + count) (or the `batch` records starting at
  * `first` when `count` is 0). A block takes chunks of 64 records: each of its
  * four wavefronts runs 16 of them forward and backward with the activations in
- * registers (every layer's result tiles are the next one's operand, as in
- * nnLayers), and leaves activations and their gradients in LDS transposed;
+ * registers (every layer's result tiles become the next one's operand,
+ * unitOrder), and leaves activations and their gradients in LDS transposed;
  * then wavefront w multiplies out the gradients of hidden units 16w..16w+15
  * (and unit tile w of W3), summed over its chunks in registers. Latency bounds
  * it (a step is one chunk a block, a chain of five products and the record
@@ -757,12 +781,13 @@ __global__ __launch_bounds__(kNnGradThreads) void k_nn_grad(const NnPacked *W, c
     }
     /* forward; lane (g, c) holds units 16m + 4g + v of record c */
     f32x4 h1[4], h2[4];
-    bf16x8 b1[2], b2[2];
+    bf16x8 b1[2], b2[2], o1[2], o2[2];
 #pragma unroll
     for (int kb = 0; kb < 2; kb++) {
 #pragma unroll
       for (int t = 0; t < 2; t++) h1[2 * kb + t] = mma16(ldOp(W->w1, kNnK1, 32 * kb + 16 * t, 0), xb, zero);
       b1[kb] = reluPackNan(h1[2 * kb], h1[2 * kb + 1]);
+      o1[kb] = unitOrder(b1[kb]);
     }
 #pragma unroll
     for (int kb = 0; kb < 2; kb++) {
@@ -770,12 +795,13 @@ __global__ __launch_bounds__(kNnGradThreads) void k_nn_grad(const NnPacked *W, c
       for (int t = 0; t < 2; t++) {
         const int m = 2 * kb + t;
         const f32x4 bias = *(const f32x4 *)&W->b2[16 * m + 4 * g];
-        h2[m] = mma16(ldOp(W->w2r, kNnHid, 16 * m, 32), b1[1], mma16(ldOp(W->w2r, kNnHid, 16 * m, 0), b1[0], bias));
+        h2[m] = mma16(ldOp(W->w2, kNnHid, 16 * m, 32), o1[1], mma16(ldOp(W->w2, kNnHid, 16 * m, 0), o1[0], bias));
       }
       b2[kb] = reluPackNan(h2[2 * kb], h2[2 * kb + 1]);
+      o2[kb] = unitOrder(b2[kb]);
     }
-    const f32x4 y = mma16(ldOp(W->w3r, kNnHid, 0, 32), b2[1],
-                          mma16(ldOp(W->w3r, kNnHid, 0, 0), b2[0], *(const f32x4 *)&W->b3[4 * g]));
+    const f32x4 y = mma16(ldOp(W->w3, kNnHid, 0, 32), o2[1],
+                          mma16(ldOp(W->w3, kNnHid, 0, 0), o2[0], *(const f32x4 *)&W->b3[4 * g]));
     /* the error: lanes 0..15 hold their record's channels; dY's operand has the channels as K */
     bf16x8 dy;
 #pragma unroll
@@ -808,9 +834,10 @@ __global__ __launch_bounds__(kNnGradThreads) void k_nn_grad(const NnPacked *W, c
         L.dh2t[u * kTs + fr] = dh;
       }
     }
+    const bf16x8 od[2] = {unitOrder(bd[0]), unitOrder(bd[1])};
 #pragma unroll
     for (int m = 0; m < 4; m++) {
-      const f32x4 d1 = mma16(ldOp(W->w2tr, kNnHid, 16 * m, 32), bd[1], mma16(ldOp(W->w2tr, kNnHid, 16 * m, 0), bd[0], zero));
+      const f32x4 d1 = mma16(ldOp(W->w2t, kNnHid, 16 * m, 32), od[1], mma16(ldOp(W->w2t, kNnHid, 16 * m, 0), od[0], zero));
 #pragma unroll
       for (int v = 0; v < 4; v++)
         L.dh1t[(16 * m + 4 * g + v) * kTs + fr] =
@@ -876,12 +903,14 @@ __device__ __forceinline__ void nnPackParam(NnPacked *W, int i, float x) {
     W->w1[(i - kOffB1) * kNnK1 + kNnIn] = h;
   } else if (i < kOffB2) {
     const int j = i - kOffW2, u = j / kNnHid, k = j % kNnHid;
+    W->w2[j] = h;
+    W->w2t[k * kNnHid + u] = h;
     W->w2r[u * kNnHid + nnRegSlot(k)] = h;
-    W->w2tr[k * kNnHid + nnRegSlot(u)] = h;
   } else if (i < kOffW3) {
     W->b2[i - kOffB2] = x;
   } else if (i < kOffB3) {
     const int j = i - kOffW3, ch = j / kNnHid, k = j % kNnHid;
+    W->w3[j] = h;
     W->w3t[k * 32 + ch] = h;
     W->w3r[ch * kNnHid + nnRegSlot(k)] = h;
   } else {
