@@ -16,7 +16,10 @@ namespace rhip {
 
 constexpr int kViewShift = 20;
 constexpr uint32_t kLocalMask = (1u << kViewShift) - 1;
-constexpr int kMaxBatchViews = 1024;  /* 3 fill ranges per view must fit the 12-bit range index */
+constexpr int kMaxBatchViews = 1024;
+constexpr int kViewFills = 3; /* fill ranges of a view: its bins, its colour, its depth */
+/* with the one of the batch's counters they must fit the range index above kViewShift */
+static_assert(kMaxBatchViews * kViewFills + 1 <= 1 << (32 - kViewShift), "fill range index");
 constexpr uint32_t kFillBlock = 4096; /* words one fill block writes */
 
 /* `n` words at `p` set to `v` */
@@ -50,6 +53,7 @@ static __global__ __launch_bounds__(256) void kb_fill(const FillRange *__restric
 static __global__ __launch_bounds__(256) void kb_vertex(const DrawParams *__restrict__ Pv, const uint32_t *__restrict__ tab) {
   const ViewBlock vb = viewBlock(Pv, tab);
   vertexBody(*vb.P, vb.local);
+  clearDrawCounts(*vb.P, vb.local); /* here and not as a fill range: a fourth one per view would not fit the range index */
 }
 
 static __global__ __launch_bounds__(256) void kb_setup(const DrawParams *__restrict__ Pv, const uint32_t *__restrict__ tab) {

@@ -165,14 +165,13 @@ int buildBatch(rhip_device d, Batch &b, const rhip_batch_config &c) {
     b.vao_refs.push_back({dd.vao, d->vao[dd.vao]->verts});
   }
 
-  /* fill ranges: per view its bins, scalars and clears, then the batch counters */
+  /* fill ranges: per view its bins and clears, then the batch counters */
   const BatchMisc M(nv);
   if ((rc = b.misc.ensure(M.bytes))) return rc;
   char *misc = b.misc.as<char>();
   std::vector<FillRange> fills;
   for (int v = 0; v < nv; v++) {
     fills.push_back({(uint32_t *)P[v].bin_count, (uint32_t)P[v].nbins, 0u});
-    fills.push_back({(uint32_t *)P[v].dcount, (uint32_t)kDrawCounts, 0u});
     const rhip_clear_states &cs = b.views[v].clear;
     const size_t px = (size_t)P[v].fb_w * P[v].fb_h * P[v].samples;
     if (cs.color_flag && P[v].color) fills.push_back({P[v].color, (uint32_t)px, clearColorWord(cs)});
@@ -201,7 +200,8 @@ int buildBatch(rhip_device d, Batch &b, const rhip_batch_config &c) {
     for (int v = 0; v < nv; v++)
       if (P[v].color) addEntries(tab, v, blocks((size_t)P[v].fb_w * P[v].fb_h, 256));
   const size_t n_res = tab.size() - o_res;
-  if (n_fill >= (1u << 31) || n_tiles >= (1u << 31)) return fail(RHIP_E_UNSUPPORTED, "batch too large");
+  if (fills.size() > (size_t)kMaxBatchViews * kViewFills + 1 || n_fill >= (1u << 31) || n_tiles >= (1u << 31))
+    return fail(RHIP_E_UNSUPPORTED, "batch too large");
 
   if ((rc = b.params.ensure(nv * sizeof(DrawParams))) || (rc = b.tabs.ensure(tab.size() * 4)) ||
       (rc = b.fills.ensure(fills.size() * sizeof(FillRange))))

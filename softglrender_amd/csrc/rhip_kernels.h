@@ -121,11 +121,16 @@ __device__ __forceinline__ void vertexBody(const DrawParams &P, int blk) {
   storeVaryings(P, i, v);
 }
 
-/* The vertex stage of one draw; it also clears the draw's bin counts and scalars, which the next stages fill. */
+/* The first block of a draw's vertex stage clears the draw's scalars, which the next stages fill. */
+__device__ __forceinline__ void clearDrawCounts(const DrawParams &P, int blk) {
+  if (blk == 0 && threadIdx.x < kDrawCounts && P.dcount) P.dcount[threadIdx.x] = 0;
+}
+
+/* The vertex stage of one draw; it also clears the draw's bin counts and scalars. */
 static __global__ __launch_bounds__(256) void k_vertex(DrawParams P) {
   vertexBody(P, blockIdx.x);
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < P.nbins; i += gridDim.x * blockDim.x) P.bin_count[i] = 0;
-  if (blockIdx.x == 0 && threadIdx.x < kDrawCounts && P.dcount) P.dcount[threadIdx.x] = 0;
+  clearDrawCounts(P, blockIdx.x);
 }
 
 /* --------------------------------------------------------------------------- block helpers */

@@ -120,3 +120,19 @@ def test_batch_rejects_what_it_cannot_run(renderer):
     rp, b, _ = replay_batched(renderer, _two_pass_stream(same_target=False))
     b.run()
     renderer.waitIdle()
+
+
+def test_batch_of_the_most_views(renderer):
+    """1,024 views, each clearing colour and depth (the most fill ranges a batch can have): identical to the checker
+    on every replay, with other draws between them."""
+    sc = scenes.scene_c4(n_scenes=3, n_views=1024, sizes=(16, 33), tri_lo=20, tri_hi=400, tex_size=16, seed=12, reads=True)
+    print("[gpu] batch of 1024 views", flush=True)
+    rp, b, reads = replay_batched(renderer, sc.stream.bytes(), layouts=sc.meta["layouts"])
+    want = _oracle(sc)
+    other = scenes.scene_c1(width=160, height=120)
+    for k in range(3):
+        print(f"[gpu] replay {k}", flush=True)
+        b.run()
+        assert_identical(run_reads(rp, reads), want, f"replay {k}")
+        replay(renderer, other.stream.bytes())
+    b.destroy()
