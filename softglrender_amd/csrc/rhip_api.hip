@@ -21,6 +21,7 @@
 #include "rhip_host.h"
 #include "rhip_launch.h"
 #include "rhip_neural.h"
+#include "rhip_ring.h"
 #include "rhip_lines.h"
 
 #include <hipcub/hipcub.hpp>

@@ -214,9 +214,6 @@ float hostPowf(float x, float y);
 int readLevel(rhip_device d, const uint8_t *src, const TexLevel &lv, int layout, void *out, uint32_t *errors);
 /* The same for `words` 4-byte words of device memory (16-byte aligned). */
 int readLinear(rhip_device d, const void *src, size_t words, void *out, uint32_t *errors);
-/* What the reads share (pinned memory, helper threads) lives while the process has devices. */
-void readDeviceAdded();
-void readDeviceGone();
 /* The IBL shaders' loop tables from the host libm's sinf / cosf. */
 void iblTablesHost(IblTables *t);
 

@@ -1,0 +1,224 @@
+/*
+ * The host side of reads (rhip_ring.h) on a stream made of one thread, without a GPU: pieces are written into their
+ * slots when the stream gets to them (or as soon as they are queued: a GPU that is far ahead of the copies), events
+ * complete in order, and allocations can be told to fail.
+ * Usage: ring_host <check>; prints "ok" and returns 0, or says what differed.
+ */
+#include <cstdarg>
+#include <cstdio>
+#include <cstdlib>
+#include <ctime>
+#include <deque>
+#include <functional>
+#include <string>
+
+#include "rhip_ring.h"
+
+/* ------------------------------------------------------------------ the stream */
+
+namespace {
+
+struct FakeStream {
+  std::mutex m;
+  std::condition_variable cv;
+  std::deque<std::function<void()>> tasks;
+  long long queued = 0, done = 0;
+  bool at_once = false;
+  FakeStream() { std::thread([this] { run(); }).detach(); }
+  void run() {
+    std::unique_lock<std::mutex> l(m);
+    for (;;) {
+      cv.wait(l, [&] { return !tasks.empty(); });
+      auto t = tasks.front();
+      tasks.pop_front();
+      l.unlock();
+      t();
+      l.lock();
+      done++;
+      cv.notify_all();
+    }
+  }
+  void push(std::function<void()> t) {
+    if (at_once) return t();
+    std::lock_guard<std::mutex> l(m);
+    tasks.push_back(std::move(t));
+    queued++;
+    cv.notify_all();
+  }
+  void wait(long long n) {
+    std::unique_lock<std::mutex> l(m);
+    cv.wait(l, [&] { return done >= n; });
+  }
+};
+FakeStream &stream() {
+  static FakeStream *s = new FakeStream();
+  return *s;
+}
+struct FakeEvent {
+  long long at = 0;
+};
+
+bool refuse_pinned = false;
+int events_left = 1 << 30; /* event creations that still succeed */
+int pinned_blocks = 0, pinned_made = 0;
+size_t pinned_bytes = 0;
+
+}  // namespace
+
+extern "C" {
+hipError_t hipHostMalloc(void **p, size_t n, unsigned int) {
+  if (refuse_pinned) return hipErrorOutOfMemory;
+  pinned_blocks++;
+  pinned_made++;
+  pinned_bytes += n;
+  return (*p = malloc(n)) ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipHostFree(void *p) {
+  pinned_blocks--;
+  free(p);
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+  if (events_left-- <= 0) return hipErrorOutOfMemory;
+  *e = (hipEvent_t) new FakeEvent();
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+  delete (FakeEvent *)e;
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+  if (!e) return hipErrorInvalidHandle;
+  FakeStream &s = stream();
+  std::lock_guard<std::mutex> l(s.m);
+  ((FakeEvent *)e)->at = s.queued;
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  stream().wait(((FakeEvent *)e)->at);
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) {
+  long long n;
+  {
+    std::lock_guard<std::mutex> l(stream().m);
+    n = stream().queued;
+  }
+  stream().wait(n);
+  return hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "error"; }
+}
+
+namespace rhip {
+std::string message;
+int fail(int code, const char *fmt, ...) {
+  char b[256];
+  va_list a;
+  va_start(a, fmt);
+  vsnprintf(b, sizeof b, fmt, a);
+  va_end(a);
+  message = b;
+  return code;
+}
+}  // namespace rhip
+
+using namespace rhip;
+
+/* ------------------------------------------------------------------ checks */
+
+namespace {
+
+std::vector<char> device_memory(size_t n, uint32_t seed) {
+  std::vector<char> v(n);
+  uint32_t x = seed * 2654435761u + 1u;
+  for (char &c : v) c = (char)((x = x * 1664525u + 1013904223u) >> 24);
+  return v;
+}
+
+/* Reads n bytes; 0 when they and the error words arrive. */
+int read(size_t n, uint32_t seed) {
+  const std::vector<char> src = device_memory(n, seed);
+  std::vector<char> out(n + 64, (char)0x5a);
+  uint32_t err[kRingErrors] = {9, 9, 9, 9};
+  const int rc = readPieces(0, nullptr, n, out.data(), err, [&](size_t at, size_t bytes, char *slot, uint32_t *errors) {
+    stream().push([=, &src] {
+      memcpy(slot, src.data() + at, bytes);
+      if (errors)
+        for (int i = 0; i < kRingErrors; i++) errors[i] = seed + i;
+    });
+    return hipSuccess;
+  });
+  if (rc) {
+    printf("%zu bytes: code %d, %s\n", n, rc, message.c_str());
+    return 1;
+  }
+  if (memcmp(out.data(), src.data(), n)) {
+    size_t at = 0;
+    while (out[at] == src[at]) at++;
+    printf("%zu bytes: differ from byte %zu on\n", n, at);
+    return 1;
+  }
+  for (size_t i = n; i < out.size(); i++)
+    if (out[i] != 0x5a) {
+      printf("%zu bytes: written past the end\n", n);
+      return 1;
+    }
+  for (int i = 0; i < kRingErrors; i++)
+    if (err[i] != seed + i) {
+      printf("%zu bytes: error word %d is %u\n", n, i, err[i]);
+      return 1;
+    }
+  return 0;
+}
+
+/* Sizes about the pieces, the line to the helpers and the ring's end, and rings walked several times, with the helper
+ * threads and without them, the stream slower and faster than the copies. */
+int checkBytes() {
+  const size_t K = kSlotBytes;
+  const size_t sizes[] = {4,     64,    K - 4,           K,          K + 4, kParallelBytes, kParallelBytes + 4, 15 * K + 8, kSlots * K,
+                          kSlots * K + 4, 17 * K, 2 * kSlots * K + 12, 53 * K + 4};
+  int bad = 0;
+  for (int own = 0; own < 2; own++) {
+    std::unique_lock<std::mutex> held;
+    std::thread other;
+    std::mutex hold;
+    std::atomic<bool> taken{false};
+    hold.lock();
+    Copiers *c = copiers();
+    if (own && c) { /* another read has the helpers */
+      other = std::thread([&] {
+        std::lock_guard<std::mutex> l(c->owner);
+        taken = true;
+        std::lock_guard<std::mutex> until(hold);
+      });
+      while (!taken) std::this_thread::yield();
+    }
+    uint32_t seed = 1;
+    for (int fast = 0; fast < 2; fast++) {
+      stream().at_once = fast;
+      for (size_t n : sizes) bad += read(n, seed++);
+      stream().at_once = false;
+    }
+    hold.unlock();
+    if (other.joinable()) other.join();
+  }
+  return bad;
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  readDeviceAdded();
+  int bad = 1;
+  if (what == "bytes") bad = checkBytes();
+  readDeviceGone();
+  if (!bad && pinned_blocks) {
+    printf("%d pinned blocks left\n", pinned_blocks);
+    bad = 1;
+  }
+  if (!bad) printf("ok\n");
+  return bad ? 1 : 0;
+}

@@ -62,7 +62,7 @@ def test_footprint_matches_checker(renderer, wrap, layout):
 
 @pytest.mark.parametrize("size", [46, 67, 129])
 def test_ibl_groups_match_checker(renderer, size):
-    """One prefiltered face of a size whose fragments are taken 2, 4 or 16 to a workgroup (the last group not full),
+    """One prefiltered face of a size whose fragments are taken 4, 8 or 16 to a workgroup (the last group not full),
     and one irradiance face (1 to a workgroup)."""
     print(f"[gpu] prefilter face of {size}^2", flush=True)
     st = S.Stream()
