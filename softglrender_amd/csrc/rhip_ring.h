@@ -154,10 +154,12 @@ struct RingLease {
     }
     r.reset(new Ring());
     r->hip_device = hip_device;
-    return r->make();
+    const int rc = r->make();
+    if (rc) r.reset(); /* half made: not for another read */
+    return rc;
   }
   ~RingLease() {
-    if (!r || !r->slots) return;
+    if (!r) return;
     Shared &s = shared();
     std::lock_guard<std::mutex> l(s.m);
     if (s.devices > 0 && s.free_rings.size() < 4) s.free_rings.push_back(std::move(r));

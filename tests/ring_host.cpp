@@ -207,6 +207,24 @@ int checkBytes() {
   return bad;
 }
 
+/* A read that could not make its ring leaves nothing behind for the next one. */
+int checkEvents() {
+  for (int k = 0; k < kSlots; k += 5) {
+    events_left = k;
+    char out[64];
+    (void)readPieces(0, nullptr, sizeof out, out, nullptr, [&](size_t, size_t, char *, uint32_t *) { return hipSuccess; });
+    events_left = 1 << 30;
+    if (pinned_blocks) {
+      printf("%d pinned blocks kept of a ring without its events\n", pinned_blocks);
+      return 1;
+    }
+    if (read(5 * kSlotBytes, 3)) return 1;
+    readDeviceGone(); /* the good ring too */
+    readDeviceAdded();
+  }
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -214,6 +232,7 @@ int main(int argc, char **argv) {
   readDeviceAdded();
   int bad = 1;
   if (what == "bytes") bad = checkBytes();
+  if (what == "events") bad = checkEvents();
   readDeviceGone();
   if (!bad && pinned_blocks) {
     printf("%d pinned blocks left\n", pinned_blocks);
