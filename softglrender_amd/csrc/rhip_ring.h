@@ -213,6 +213,8 @@ int readPieces(int hip_device, hipStream_t stream, size_t bytes, void *out, uint
   while (issued < std::min(pieces, kSlots) && he == hipSuccess) issue();
   if (he != hipSuccess) return give_up();
 
+  /* the work queued before the read is waited for here, and only then are helpers woken: they never spin through it */
+  if ((he = hipEventSynchronize(R.ev[0])) != hipSuccess) return give_up();
   Copiers *C = bytes > kParallelBytes ? copiers() : nullptr;
   std::unique_lock<std::mutex> own;
   if (C) own = std::unique_lock<std::mutex>(C->owner, std::try_to_lock);

@@ -4,6 +4,7 @@
  * complete in order, and allocations can be told to fail.
  * Usage: ring_host <check>; prints "ok" and returns 0, or says what differed.
  */
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -225,6 +226,29 @@ int checkEvents() {
   return 0;
 }
 
+/* While the stream still works on what was queued before the read, nothing of the read takes processor time. */
+int checkIdle() {
+  bool helpers = copiers() != nullptr;
+  for (int k = 0; k < 2; k++) {
+    stream().push([] { std::this_thread::sleep_for(std::chrono::milliseconds(400)); });
+    const size_t n = 8 * kSlotBytes;
+    const std::vector<char> src = device_memory(n, 1);
+    std::vector<char> out(n);
+    const clock_t c0 = clock(); /* of all threads */
+    const int rc = readPieces(0, nullptr, n, out.data(), nullptr, [&](size_t at, size_t bytes, char *slot, uint32_t *) {
+      stream().push([=, &src] { memcpy(slot, src.data() + at, bytes); });
+      return hipSuccess;
+    });
+    const double ms = (clock() - c0) * 1e3 / CLOCKS_PER_SEC;
+    if (rc || out != src) return 1;
+    if (ms > 200) { /* 16 MiB copied: a few; one thread that spins: 400 */
+      printf("%.0f ms of processor time in a read that waited 400 ms (helpers: %d)\n", ms, (int)helpers);
+      return 1;
+    }
+  }
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -233,6 +257,7 @@ int main(int argc, char **argv) {
   int bad = 1;
   if (what == "bytes") bad = checkBytes();
   if (what == "events") bad = checkEvents();
+  if (what == "idle") bad = checkIdle();
   readDeviceGone();
   if (!bad && pinned_blocks) {
     printf("%d pinned blocks left\n", pinned_blocks);

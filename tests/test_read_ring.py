@@ -19,7 +19,7 @@ def ring_host(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["bytes", "events"])
+@pytest.mark.parametrize("check", ["bytes", "events", "idle"])
 def test_ring(ring_host, check):
     r = subprocess.run([ring_host, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
