@@ -46,21 +46,6 @@ int fail(int code, const char *fmt, ...) {
 
 namespace {
 
-/* Texel index in a level's storage order (host side of texelIndex). */
-size_t hostTexelIndex(const TexLevel &l, int layout, int x, int y) {
-  if (layout == LAYOUT_TILED)
-    return ((size_t)((uint32_t)(y >> 2) * l.tiles_x + (uint32_t)(x >> 2)) << 4) + ((y & 3) << 2) + (x & 3);
-  if (layout == LAYOUT_MORTON) {
-    uint32_t r = (uint32_t)(x & 31) | ((uint32_t)(y & 31) << 16);
-    r = (r | (r << 4)) & 0x0f0f0f0fu;
-    r = (r | (r << 2)) & 0x33333333u;
-    r = (r | (r << 1)) & 0x55555555u;
-    r = (r | (r >> 15)) & 0xffffu;
-    return ((size_t)((uint32_t)(y >> 5) * l.tiles_x + (uint32_t)(x >> 5)) << 10) + r;
-  }
-  return (size_t)y * l.w + x;
-}
-
 int levelCount(int w, int h) { return (int)std::floor(std::log2((double)std::max(w, h))) + 1; }
 
 /* Allocates storage for every level of every layer in the texture's layout. */

@@ -47,15 +47,19 @@ __global__ __launch_bounds__(256) void k_read_words(const uint32_t *src, TexLeve
 int readWords(rhip_device d, const void *src, const TexLevel *lv, int layout, size_t words, void *out,
               uint32_t *errors) {
   const TexLevel level = lv ? *lv : TexLevel{};
-  return readPieces(d->hip_device, d->stream, words * 4, out, errors,
-                    [&](size_t at, size_t bytes, char *slot, uint32_t *errors_out) {
-                      const size_t n = bytes / 4;
-                      const unsigned grid = std::max(1u, std::min(blocks(n, 1024), 256u));
-                      k_read_words<<<grid, 256, 0, d->stream>>>((const uint32_t *)src, level, layout, at / 4, n,
-                                                                (uint32_t *)slot, errors_out ? d->errors : nullptr,
-                                                                errors_out);
-                      return hipGetLastError();
-                    });
+  const int rc = readPieces(d->hip_device, d->stream, words * 4, out, errors,
+                            [&](size_t at, size_t bytes, char *slot, uint32_t *errors_out) {
+                              const size_t n = bytes / 4;
+                              const unsigned grid = std::max(1u, std::min(blocks(n, 1024), 256u));
+                              k_read_words<<<grid, 256, 0, d->stream>>>((const uint32_t *)src, level, layout, at / 4, n,
+                                                                        (uint32_t *)slot,
+                                                                        errors_out ? d->errors : nullptr, errors_out);
+                              return hipGetLastError();
+                            });
+  if (rc != kNoPinned) return rc;
+  if (layout == LAYOUT_LINEAR) return readPageable(d->stream, src, words, out, d->errors, errors);
+  return readPageable(d->stream, src, (size_t)level.inner_w * level.inner_h, level.w, level.h, out, d->errors, errors,
+                      [&](int x, int y) { return hostTexelIndex(level, layout, x, y); });
 }
 
 }  // namespace

@@ -27,25 +27,28 @@ int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 
 constexpr size_t kSlotBytes = (size_t)1 << 20;
 constexpr int kSlots = 16;
+constexpr size_t kSmallBytes = (size_t)256 << 10; /* reads up to here take a ring of one slot of this size */
 constexpr size_t kParallelBytes = (size_t)2 << 20; /* larger reads are copied out by the helpers */
 constexpr int kRingErrors = 4;                     /* the device's error words come along with the first piece */
+constexpr int kNoPinned = 1;                       /* readPieces: pinned memory was refused, nothing was queued */
 
 /* ------------------------------------------------------------------ pinned rings
  * One per read in progress, shared by the process's devices: a read takes a
  * free one or makes one; they are freed with the last device. */
 struct Ring {
-  int hip_device = 0;    /* its events belong to this GPU */
-  char *slots = nullptr; /* kSlots x kSlotBytes, then the error words */
+  int hip_device = 0; /* its events belong to this GPU */
+  int count = 0;      /* slots */
+  size_t slot_bytes = 0;
+  char *slots = nullptr; /* the slots, then the error words */
   hipEvent_t ev[kSlots] = {};
-  uint32_t *errors() const { return (uint32_t *)(slots + kSlots * kSlotBytes); }
-  int make() {
-    if (hipHostMalloc((void **)&slots, kSlots * kSlotBytes + 4096, hipHostMallocDefault) != hipSuccess) {
-      slots = nullptr;
-      return fail(RHIP_E_OOM, "pinned memory for reads");
-    }
-    for (hipEvent_t &e : ev)
-      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return fail(RHIP_E_HIP, "read events");
-    return RHIP_OK;
+  uint32_t *errors() const { return (uint32_t *)(slots + count * slot_bytes); }
+  /* false where pinned memory or an event is refused (its error is not left for a later call to report) */
+  bool make() {
+    bool ok = hipHostMalloc((void **)&slots, count * slot_bytes + 4096, hipHostMallocDefault) == hipSuccess;
+    if (!ok) slots = nullptr;
+    for (int i = 0; i < count && ok; i++) ok = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    return ok;
   }
   ~Ring() {
     for (hipEvent_t e : ev)
@@ -126,6 +129,7 @@ struct Copiers {
   }
 };
 
+constexpr int kKeptRings = 4; /* of either size: 65 MiB of pinned memory at most */
 struct Shared {
   std::mutex m;
   std::vector<std::unique_ptr<Ring>> free_rings;
@@ -140,29 +144,33 @@ inline Shared &shared() {
 
 struct RingLease {
   std::unique_ptr<Ring> r;
-  int take(int hip_device) {
+  bool take(int hip_device, bool small) {
+    const int count = small ? 1 : kSlots;
     Shared &s = shared();
     {
       std::lock_guard<std::mutex> l(s.m);
       for (auto &f : s.free_rings)
-        if (f->hip_device == hip_device) {
+        if (f->hip_device == hip_device && f->count == count) {
           r = std::move(f);
           f = std::move(s.free_rings.back());
           s.free_rings.pop_back();
-          return RHIP_OK;
+          return true;
         }
     }
     r.reset(new Ring());
     r->hip_device = hip_device;
-    const int rc = r->make();
-    if (rc) r.reset(); /* half made: not for another read */
-    return rc;
+    r->count = count;
+    r->slot_bytes = small ? kSmallBytes : kSlotBytes;
+    if (!r->make()) r.reset(); /* half made: not for another read */
+    return r != nullptr;
   }
   ~RingLease() {
     if (!r) return;
     Shared &s = shared();
     std::lock_guard<std::mutex> l(s.m);
-    if (s.devices > 0 && s.free_rings.size() < 4) s.free_rings.push_back(std::move(r));
+    const auto same = [&](const std::unique_ptr<Ring> &f) { return f->count == r->count; };
+    if (s.devices > 0 && std::count_if(s.free_rings.begin(), s.free_rings.end(), same) < kKeptRings)
+      s.free_rings.push_back(std::move(r));
   }
 };
 
@@ -185,14 +193,13 @@ inline Copiers *copiers() {
 
 /* `bytes` bytes of device memory to out, piece by piece: issue(at, n, slot, errors) queues on `stream` what puts bytes
  * [at, at + n) into a slot, and the device's error words to `errors` where that is not null. `errors` (kRingErrors
- * words, may be null) gets those. */
+ * words, may be null) gets those. kNoPinned where no ring is to be had. */
 template <typename Issue>
 int readPieces(int hip_device, hipStream_t stream, size_t bytes, void *out, uint32_t *errors, Issue issue_piece) {
   RingLease lease;
-  int rc = lease.take(hip_device);
-  if (rc) return rc;
+  if (!lease.take(hip_device, bytes <= kSmallBytes)) return kNoPinned;
   Ring &R = *lease.r;
-  const int pieces = (int)((bytes + kSlotBytes - 1) / kSlotBytes);
+  const int pieces = (int)((bytes + kSlotBytes - 1) / kSlotBytes); /* of a small read: one */
   if (errors) memset(errors, 0, kRingErrors * 4);
   if (!pieces) return RHIP_OK;
   hipError_t he = hipSuccess;
@@ -249,6 +256,30 @@ int readPieces(int hip_device, hipStream_t stream, size_t bytes, void *out, uint
     if (he != hipSuccess) return give_up();
   }
   if (errors) memcpy(errors, R.errors(), kRingErrors * 4);
+  return RHIP_OK;
+}
+
+/* A read without pinned memory: `words` words of device memory to out, and the device's error words. */
+inline int readPageable(hipStream_t stream, const void *src, size_t words, void *out, const uint32_t *dev_errors,
+                        uint32_t *errors) {
+  hipError_t he = hipMemcpyAsync(out, src, words * 4, hipMemcpyDeviceToHost, stream);
+  if (he == hipSuccess && errors)
+    he = hipMemcpyAsync(errors, dev_errors, kRingErrors * 4, hipMemcpyDeviceToHost, stream);
+  const hipError_t se = hipStreamSynchronize(stream);
+  if (he == hipSuccess) he = se;
+  return he == hipSuccess ? RHIP_OK : fail(RHIP_E_HIP, "read: %s", hipGetErrorString(he));
+}
+
+/* The same for an image of w x h texels stored in `stored` words, texel (x, y) at index(x, y). */
+template <typename Index>
+int readPageable(hipStream_t stream, const void *src, size_t stored, int w, int h, void *out, const uint32_t *dev_errors,
+                 uint32_t *errors, Index index) {
+  std::vector<uint32_t> tmp(stored);
+  const int rc = readPageable(stream, src, stored, tmp.data(), dev_errors, errors);
+  if (rc) return rc;
+  uint32_t *o = (uint32_t *)out;
+  for (int y = 0; y < h; y++)
+    for (int x = 0; x < w; x++) *o++ = tmp[index(x, y)];
   return RHIP_OK;
 }
 

@@ -59,18 +59,18 @@ struct FakeEvent {
   long long at = 0;
 };
 
-bool refuse_pinned = false;
+size_t pinned_limit = (size_t)-1; /* larger allocations are refused */
+hipError_t last_error = hipSuccess;
 int events_left = 1 << 30; /* event creations that still succeed */
-int pinned_blocks = 0, pinned_made = 0;
+int pinned_blocks = 0;
 size_t pinned_bytes = 0;
 
 }  // namespace
 
 extern "C" {
 hipError_t hipHostMalloc(void **p, size_t n, unsigned int) {
-  if (refuse_pinned) return hipErrorOutOfMemory;
+  if (n > pinned_limit) return last_error = hipErrorOutOfMemory;
   pinned_blocks++;
-  pinned_made++;
   pinned_bytes += n;
   return (*p = malloc(n)) ? hipSuccess : hipErrorOutOfMemory;
 }
@@ -80,7 +80,7 @@ hipError_t hipHostFree(void *p) {
   return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
-  if (events_left-- <= 0) return hipErrorOutOfMemory;
+  if (events_left-- <= 0) return last_error = hipErrorOutOfMemory;
   *e = (hipEvent_t) new FakeEvent();
   return hipSuccess;
 }
@@ -108,7 +108,15 @@ hipError_t hipStreamSynchronize(hipStream_t) {
   stream().wait(n);
   return hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = last_error;
+  last_error = hipSuccess;
+  return e;
+}
+hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, hipMemcpyKind, hipStream_t) {
+  stream().push([=] { memcpy(to, from, n); });
+  return hipSuccess;
+}
 const char *hipGetErrorString(hipError_t) { return "error"; }
 }
 
@@ -143,7 +151,7 @@ int read(size_t n, uint32_t seed) {
   const std::vector<char> src = device_memory(n, seed);
   std::vector<char> out(n + 64, (char)0x5a);
   uint32_t err[kRingErrors] = {9, 9, 9, 9};
-  const int rc = readPieces(0, nullptr, n, out.data(), err, [&](size_t at, size_t bytes, char *slot, uint32_t *errors) {
+  int rc = readPieces(0, nullptr, n, out.data(), err, [&](size_t at, size_t bytes, char *slot, uint32_t *errors) {
     stream().push([=, &src] {
       memcpy(slot, src.data() + at, bytes);
       if (errors)
@@ -151,6 +159,10 @@ int read(size_t n, uint32_t seed) {
     });
     return hipSuccess;
   });
+  if (rc == kNoPinned) {
+    const uint32_t dev_errors[kRingErrors] = {seed, seed + 1, seed + 2, seed + 3};
+    rc = readPageable(nullptr, src.data(), n / 4, out.data(), dev_errors, err);
+  }
   if (rc) {
     printf("%zu bytes: code %d, %s\n", n, rc, message.c_str());
     return 1;
@@ -178,7 +190,7 @@ int read(size_t n, uint32_t seed) {
  * threads and without them, the stream slower and faster than the copies. */
 int checkBytes() {
   const size_t K = kSlotBytes;
-  const size_t sizes[] = {4,     64,    K - 4,           K,          K + 4, kParallelBytes, kParallelBytes + 4, 15 * K + 8, kSlots * K,
+  const size_t sizes[] = {4,     64,    kSmallBytes, kSmallBytes + 4, K - 4,           K,          K + 4, kParallelBytes, kParallelBytes + 4, 15 * K + 8, kSlots * K,
                           kSlots * K + 4, 17 * K, 2 * kSlots * K + 12, 53 * K + 4};
   int bad = 0;
   for (int own = 0; own < 2; own++) {
@@ -212,8 +224,8 @@ int checkBytes() {
 int checkEvents() {
   for (int k = 0; k < kSlots; k += 5) {
     events_left = k;
-    char out[64];
-    (void)readPieces(0, nullptr, sizeof out, out, nullptr, [&](size_t, size_t, char *, uint32_t *) { return hipSuccess; });
+    std::vector<char> out(2 * kSlotBytes);
+    (void)readPieces(0, nullptr, out.size(), out.data(), nullptr, [&](size_t, size_t, char *, uint32_t *) { return hipSuccess; });
     events_left = 1 << 30;
     if (pinned_blocks) {
       printf("%d pinned blocks kept of a ring without its events\n", pinned_blocks);
@@ -249,6 +261,38 @@ int checkIdle() {
   return 0;
 }
 
+/* Where pinned memory is refused, reads copy through pageable memory, every layout, and leave no error behind; a small
+ * read asks for little of it. */
+int checkRefused() {
+  if (read(64, 1)) return 1;
+  if (pinned_bytes > 512 << 10) {
+    printf("%zu bytes pinned for a read of 64\n", pinned_bytes);
+    return 1;
+  }
+  readDeviceGone();
+  readDeviceAdded();
+  for (size_t limit : {(size_t)0, (size_t)1 << 20}) {
+    pinned_limit = limit;
+    for (size_t n : {(size_t)4, (size_t)64, kSlotBytes + 4, 5 * kSlotBytes})
+      if (read(n, (uint32_t)n)) return 1;
+    if (last_error != hipSuccess) {
+      printf("the refused allocation's error is left for the next call\n");
+      return 1;
+    }
+  }
+  /* a 6 x 5 image stored column by column, with a column of padding */
+  const uint32_t stored[35] = {0,  1,  2,  3,  4,  5,  6,  7,  8,  9,  10, 11, 12, 13, 14, 15, 16, 17,
+                               18, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30, 31, 32, 33, 34};
+  const uint32_t dev_errors[kRingErrors] = {4, 3, 2, 1};
+  uint32_t out[31], errors[kRingErrors];
+  out[30] = 77;
+  if (readPageable(nullptr, stored, 35, 6, 5, out, dev_errors, errors, [](int x, int y) { return (size_t)x * 5 + y; }))
+    return 1;
+  for (int i = 0; i < 30; i++)
+    if (out[i] != (uint32_t)(i % 6 * 5 + i / 6)) return printf("pageable: texel %d is %u\n", i, out[i]), 1;
+  return out[30] != 77 || memcmp(errors, dev_errors, sizeof errors);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -258,6 +302,7 @@ int main(int argc, char **argv) {
   if (what == "bytes") bad = checkBytes();
   if (what == "events") bad = checkEvents();
   if (what == "idle") bad = checkIdle();
+  if (what == "refused") bad = checkRefused();
   readDeviceGone();
   if (!bad && pinned_blocks) {
     printf("%d pinned blocks left\n", pinned_blocks);

@@ -19,7 +19,7 @@ def ring_host(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["bytes", "events", "idle"])
+@pytest.mark.parametrize("check", ["bytes", "events", "idle", "refused"])
 def test_ring(ring_host, check):
     r = subprocess.run([ring_host, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
