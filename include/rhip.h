@@ -157,9 +157,10 @@ int rhip_draw(rhip_device dev, const rhip_draw_desc *draw);
  * static device buffer of rhip_draw_noalloc_capacity() bytes (64 MiB) that
  * every call on one GPU shares and that keeps the last call's contents: calls
  * that overlap on one GPU (two devices' streams, or another thread) race. A
- * draw whose worst-case arena exceeds it fails with RHIP_E_UNSUPPORTED (about
- * 4k triangles at 640x480 with 4x MSAA fit), and so does a draw of points or
- * lines (their fragment list is sized at draw time). Results equal rhip_draw's. */
+ * draw whose worst-case arena, counted with room for 12 clipped vertices a
+ * triangle, exceeds it fails with RHIP_E_UNSUPPORTED (about 4k triangles at
+ * 640x480 with 4x MSAA fit), and so does a draw of points or lines (their
+ * fragment list is sized at draw time). Results equal rhip_draw's. */
 int rhip_draw_noalloc(rhip_device dev, const rhip_draw_desc *draw);
 size_t rhip_draw_noalloc_capacity(void);
 int rhip_end_render_pass(rhip_device dev);                                            /* endRenderPass (Renderer.h:57) */

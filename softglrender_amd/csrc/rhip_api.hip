@@ -416,16 +416,12 @@ size_t carveArenas(DrawParams &P, const DrawShape &sh, char *base) {
     return p;
   };
   const size_t V = sh.V, T = sh.T, vcap = V + T * kMaxClipVerts, pcap = T * (1 + kMaxFans);
-  const int nblk = P.nblk;
   P.clip = (float4 *)take(vcap * 16);
   P.frag = (float4 *)take(vcap * 16);
   P.mask = (int *)take(vcap * 4);
   P.vary = (float *)take(vcap * P.vary_stride * 4);
   P.clip_poly = (int *)take(T * (kMaxPoly + 1) * 4);
   P.clip_list = (int *)take(T * 4);
-  /* room that clipping no longer uses: what a draw needs, and so what rhip_draw_noalloc takes, stays what it was */
-  take(T * kMaxClipVerts * sh.stride);
-  take(((size_t)nblk * 3 + (nblk + 63) / 64) * 4);
   P.dcount = (int *)take(64);
   P.prims = (PrimSetup *)take(pcap * sizeof(PrimSetup));
   P.bin_count = (int *)take(((size_t)P.nbins * 3 + 1) * 4);
@@ -954,6 +950,15 @@ int drawPointsLines(rhip_device d, DrawParams &P, const DrawShape &sh, bool no_a
   return RHIP_OK;
 }
 
+/* The size of a draw that rhip_draw_noalloc holds against its capacity: the arena, and for each triangle the vertices
+ * that clipping may make and three words for every 256. No stage keeps the latter two in memory; they are counted so
+ * that the draws this call takes and refuses are a fixed set. */
+size_t noallocSize(const DrawParams &P, const DrawShape &sh, size_t arena) {
+  auto whole = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  const size_t nblk = (size_t)P.nblk;
+  return arena + whole(sh.T * kMaxClipVerts * sh.stride) + whole((nblk * 3 + (nblk + 63) / 64) * 4);
+}
+
 /* One draw (RendererSoft::draw, RendererSoft.cpp:136-164) with its arena in
  * the device's grow-only buffer, or, for no_alloc, in the library's static
  * scratch of kScratchBytes. */
@@ -979,11 +984,12 @@ int drawOne(rhip_device d, const rhip_draw_desc *dd, bool no_alloc) {
   if (sh.lines) return drawPointsLines(d, P, sh, no_alloc);
   const size_t need = carveArenas(P, sh, nullptr);
   if (no_alloc) {
-    if (need > kScratchBytes)
+    const size_t size = noallocSize(P, sh, need);
+    if (size > kScratchBytes)
       return fail(RHIP_E_UNSUPPORTED,
                   "rhip_draw_noalloc: this draw needs %zu bytes of scratch, more than the %zu the library holds "
                   "(%zu vertices, %zu triangles, %dx%d x%d samples); use rhip_draw",
-                  need, kScratchBytes, sh.V, sh.T, P.fb_w, P.fb_h, P.samples);
+                  size, kScratchBytes, sh.V, sh.T, P.fb_w, P.fb_h, P.samples);
     if (!d->scratch) return fail(RHIP_E_HIP, "rhip_draw_noalloc: no scratch address for this device");
     carveArenas(P, sh, d->scratch);
   } else {
