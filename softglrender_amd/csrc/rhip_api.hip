@@ -852,7 +852,9 @@ int drawPointsLines(rhip_device d, DrawParams &P, const DrawShape &sh, bool no_a
   };
   PlUnit *units = nullptr;
   unsigned long long *count = nullptr, *offset = nullptr;
-  int *head = nullptr, *next = nullptr; /* per vertex, its point units (a linked list) */
+  /* point units by vertex: per vertex (and for all, at V) their number, per vertex where they start in `sorted` */
+  int *vcount = nullptr, *vstart = nullptr, *sorted = nullptr;
+  int2 *where = nullptr;
   void *tmp = nullptr;
   for (int pass = 0; pass < 2; pass++) {
     off = 0;
@@ -863,8 +865,12 @@ int drawPointsLines(rhip_device d, DrawParams &P, const DrawShape &sh, bool no_a
     units = (PlUnit *)take((size_t)U * sizeof(PlUnit));
     count = (unsigned long long *)take((size_t)(U + 1) * 8);
     offset = (unsigned long long *)take((size_t)(U + 1) * 8);
-    head = (int *)take((size_t)V * 4);
-    next = (int *)take((size_t)U * 4);
+    if (points) {
+      vcount = (int *)take((size_t)(V + 1) * 4);
+      vstart = (int *)take((size_t)V * 4);
+      where = (int2 *)take((size_t)U * 8);
+      sorted = (int *)take((size_t)U * 4);
+    }
     tmp = take(scan_tmp);
     if (pass == 0) {
       int rc = d->arena.ensure(off);
@@ -872,20 +878,23 @@ int drawPointsLines(rhip_device d, DrawParams &P, const DrawShape &sh, bool no_a
       base = d->arena.as<char>();
     }
   }
+  if (points) { /* cleared by the vertex stage, as a triangle draw's bins are */
+    P.bin_count = vcount;
+    P.nbins = (int)V + 1;
+  }
   { Timer tm(d, "k_vertex"); RHIP_LAUNCH(k_vertex, std::max(blocks((size_t)V, 256), 1u), 256, s, P); }
   unsigned long long total = 0;
   if (U > 0) {
     const unsigned g = blocks((size_t)U, 256);
-    if (points)
-      RHIP_LAUNCH(k_fill2_u32, std::min(blocks((size_t)V, 1024), 1024u), 256, s, (uint32_t *)head, (size_t)V, 0xffffffffu,
-                  (uint32_t *)nullptr, (size_t)0, 0u);
     {
       Timer tm(d, "k_pl_units");
-      RHIP_LAUNCH(k_pl_units, blocks((size_t)U + 1, 256), 256, s, P, units, U, count, head, next, has_colour ? 1 : 0);
+      RHIP_LAUNCH(k_pl_units, blocks((size_t)U + 1, 256), 256, s, P, units, U, count, vcount, where, has_colour ? 1 : 0);
     }
     if (points) {
+      RHIP_LAUNCH(k_pl_place, blocks((size_t)V, 1024), 1024, s, vcount, vstart, (int)V);
+      RHIP_LAUNCH(k_pl_sort, g, 256, s, where, vstart, U, sorted);
       Timer tm(d, "k_pl_points");
-      RHIP_LAUNCH(k_pl_points, g, 256, s, P, units, head, next, U, count, has_colour ? 1 : 0);
+      RHIP_LAUNCH(k_pl_points, g, 256, s, P, units, vcount, vstart, sorted, count, has_colour ? 1 : 0);
     }
     size_t t = scan_tmp;
     HIPCHK(hipcub::DeviceScan::ExclusiveSum(tmp, t, count, offset, (size_t)U + 1, s));

@@ -13,11 +13,12 @@
  *                ("unit"): assembly, clipping (new vertices re-run the vertex
  *                shader), face culling of triangles in point/line mode; a line
  *                counts its fragments here
+ *   k_pl_place, k_pl_sort  the point units of each vertex side by side
  *   k_pl_points  the reference writes each rasterized point's last pixel back
  *                into its vertex's screen position, so the k-th rasterization
  *                of a vertex starts where the (k-1)-th ended; each point unit
- *                finds its place in its vertex's list of units (k_pl_units
- *                makes the lists), replays that chain and counts its fragments
+ *                finds its rank among its vertex's units, replays that chain
+ *                and counts its fragments
  *   (scan)       fragment offsets per unit: the fragments' draw order
  *   k_pl_emit    every unit writes its fragments (pixel key, depth, colour) at
  *                its offset, in the reference's loop order
@@ -247,9 +248,10 @@ __device__ void plUnitSetupRaw(const DrawParams &P, int u, PlUnit &U) {
 /* One thread sets up a unit; a line's fragments (every step is a point of the
  * line's width) are then counted by 16 lanes, a step each, for lines wider than
  * a pixel; a step of width 1 is always one fragment ([c, c + 1) for a whole
- * number c below 2^24, exactly). A point goes into its vertex's list. */
+ * number c below 2^24, exactly). A point is counted at its vertex; `where` gets
+ * its vertex (-1: no point) and its place there, in no order. */
 static __global__ __launch_bounds__(256) void k_pl_units(DrawParams P, PlUnit *units, long long nunits,
-                                                        unsigned long long *count, int *head, int *next,
+                                                        unsigned long long *count, int *vcount, int2 *where,
                                                         int has_colour) {
   const long long u = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (u == nunits) count[u] = 0; /* the scan's end: the total */
@@ -259,7 +261,7 @@ static __global__ __launch_bounds__(256) void k_pl_units(DrawParams P, PlUnit *u
   if (mine) {
     plUnitSetup(P, (int)u, U);
     units[u] = U;
-    if (U.kind == kPlPoint) next[u] = atomicExch(&head[U.vertex], (int)u);
+    if (where) where[u] = U.kind == kPlPoint ? make_int2(U.vertex, atomicAdd(&vcount[U.vertex], 1)) : make_int2(-1, 0);
   }
   const bool line = has_colour && U.kind == kPlLine;
   const float width = P.st.lineWidth;
@@ -287,18 +289,56 @@ static __global__ __launch_bounds__(256) void k_pl_units(DrawParams P, PlUnit *u
   if (mine) count[u] = n;
 }
 
+/* Where each vertex's point units start in `sorted`: any order of the vertices does, so a workgroup takes room for its
+ * 1,024 with one atomic on vcount[nverts] (one per wavefront took 179 us for a million vertices, on one address). */
+static __global__ __launch_bounds__(1024) void k_pl_place(int *vcount, int *vstart, int nverts) {
+  __shared__ int s_wave[16], s_base;
+  const int v = blockIdx.x * blockDim.x + threadIdx.x, w = threadIdx.x >> 6;
+  const int n = v < nverts ? vcount[v] : 0;
+  const int inc = waveInclusiveScan(n);
+  if ((threadIdx.x & 63) == 63) s_wave[w] = inc;
+  __syncthreads();
+  int before = 0, all = 0;
+  for (int k = 0; k < 16; k++) {
+    before += k < w ? s_wave[k] : 0;
+    all += s_wave[k];
+  }
+  if (threadIdx.x == 0) s_base = all ? atomicAdd(&vcount[nverts], all) : 0;
+  __syncthreads();
+  if (v < nverts) vstart[v] = s_base + before + inc - n;
+}
+static __global__ __launch_bounds__(256) void k_pl_sort(const int2 *where, const int *vstart, long long nunits, int *sorted) {
+  const long long u = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= nunits) return;
+  const int2 w = where[u];
+  if (w.x >= 0) sorted[vstart[w.x] + w.y] = (int)u;
+}
+
 /* A point unit is the r-th rasterization of its vertex, r the vertex's units
  * before it. Each rasterization moves the vertex's screen position to the last
  * pixel it wrote (RendererSoft.cpp:637-661 writes x, y into v->fragPos), so unit
- * r starts r moves on. */
-static __global__ __launch_bounds__(256) void k_pl_points(DrawParams P, PlUnit *units, const int *head, const int *next,
-                                                         long long nunits, unsigned long long *count, int has_colour) {
-  const long long u = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= nunits) return;
+ * r starts r moves on. Lane j takes the unit in place j, so that the lanes of a
+ * wavefront have few vertices: all m units of one are compared with all m by
+ * loads that the lanes share and that wait for nothing. A linked list per vertex,
+ * walked by each of its units, needs no places but a chain of m loads a lane. */
+static __global__ __launch_bounds__(256) void k_pl_points(DrawParams P, PlUnit *units, const int *vcount, const int *vstart,
+                                                         const int *sorted, unsigned long long *count, int has_colour) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= vcount[P.nverts]) return;
+  const int u = sorted[j];
   PlUnit &U = units[u];
-  if (U.kind != kPlPoint) return;
-  int r = 0;
-  for (int j = head[U.vertex]; j >= 0; j = next[j]) r += j < (int)u ? 1 : 0;
+  struct __attribute__((packed, aligned(4))) Four {
+    int i[4];
+  };
+  const int m = vcount[U.vertex];
+  const int *s = sorted + vstart[U.vertex];
+  int r = 0, i = 0;
+#pragma unroll 4
+  for (; i + 4 <= m; i += 4) {
+    const Four f = *(const Four *)(s + i);
+    r += (f.i[0] < u) + (f.i[1] < u) + (f.i[2] < u) + (f.i[3] < u);
+  }
+  for (; i < m; i++) r += s[i] < u ? 1 : 0;
   float px = U.a.x, py = U.a.y;
   const float size = P.pl_point_size;
   int x0, x1, y0, y1;

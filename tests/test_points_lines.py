@@ -159,3 +159,27 @@ def test_hip_small_cases(renderer):
                _screen_scene([(10.3, 7.8)], [0], S.PRIM_POINT, msaa=True),
                _screen_scene([(10.3, 7.8)], [0], S.PRIM_POINT, colour=False)):
         _assert_identical(_hip(renderer, sc), _checker(sc), "small")
+
+
+def _spread(count, w, h, seed):
+    rng = np.random.default_rng(seed)
+    return np.stack([rng.uniform(1, w - 1, count), rng.uniform(1, h - 1, count)], 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("verts,units,every", [(1, 1, 1), (1, 3000, 1), (1023, 4097, 7), (1024, 1024, 3), (1025, 2500, 64),
+                                               (3000, 9000, 2)])
+def test_hip_points_that_share_a_vertex(renderer, verts, units, every):
+    """Point lists in which every `every`-th point is vertex 0 and the others come in a shuffled order, some several
+    times: each rasterization of a vertex starts where its last one ended, so that their order shows."""
+    rng = np.random.default_rng(units)
+    idx = np.resize(rng.permutation(verts), units)
+    idx[::every] = 0
+    for size in (1.0, 2.6):
+        print(f"[gpu] {units} points on {verts} vertices, size {size}", flush=True)
+        sc = _screen_scene(_spread(verts, 61, 47, verts), idx, S.PRIM_POINT, point_size=size, w=61, h=47)
+        _assert_identical(_hip(renderer, sc), _checker(sc), f"{verts} {units} {size}")
+    tri = idx[: units - units % 3]
+    if len(tri):
+        sc = _screen_scene(_spread(verts, 61, 47, verts), tri, S.PRIM_TRIANGLE, mode=S.POLY_POINT, point_size=1.7, w=61, h=47)
+        _assert_identical(_hip(renderer, sc), _checker(sc), f"triangles {verts} {units}")
