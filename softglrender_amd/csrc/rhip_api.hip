@@ -1323,6 +1323,7 @@ int rhip_neural_train(rhip_device d, long long first, long long count, int steps
   auto &n = d->nn;
   std::vector<double> lh;
   double *dl = nullptr;
+  const CallBuf kept{n.losses};
   if (losses && steps > 0) { /* every step writes its own */
     if ((rc = n.losses.ensure(steps * sizeof(double)))) return rc;
     dl = n.losses.as<double>();
@@ -1375,6 +1376,7 @@ int rhip_neural_evaluate(rhip_device d, long long first, long long count, int ma
   if (count > INT32_MAX) return fail(RHIP_E_INVALID, "too many records");
   auto &n = d->nn;
   float *dout = nullptr;
+  const CallBuf kept{n.outputs};
   if (outputs) {
     if ((rc = n.outputs.ensure((size_t)count * 3 * sizeof(float)))) return rc;
     dout = n.outputs.as<float>();

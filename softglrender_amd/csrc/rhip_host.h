@@ -47,8 +47,20 @@ struct DevBuf {
   T *as() const {
     return (T *)p;
   }
-  ~DevBuf() {
+  void release() {
     if (p) hipFree(p);
+    p = nullptr;
+    cap = 0;
+  }
+  ~DevBuf() { release(); }
+};
+
+/* A call's use of a buffer that the device keeps for the next one only up to kKeptBytes. */
+struct CallBuf {
+  static constexpr size_t kKeptBytes = (size_t)16 << 20;
+  DevBuf &b;
+  ~CallBuf() {
+    if (b.cap > kKeptBytes) b.release();
   }
 };
 
@@ -135,8 +147,8 @@ struct rhip_device_s {
     int step = 0;
     bool ready = false;
     rhip::DevBuf records;
-    rhip::DevBuf outputs; /* an evaluation's network outputs */
-    rhip::DevBuf losses;  /* a training run's, one per step */
+    rhip::DevBuf outputs; /* an evaluation's network outputs (CallBuf) */
+    rhip::DevBuf losses;  /* a training run's, one per step (CallBuf) */
     long long rec_cap = 0;
     unsigned long long *rec_count = nullptr;
     bool capturing = false;

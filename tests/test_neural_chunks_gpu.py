@@ -1,9 +1,12 @@
 """The learned shader's gradient, evaluation and training at record counts on either side of their chunks (64 records,
 1,024 blocks of them), against the numpy network."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from oracle import nn_ref as nn
+from softglrender_amd import _lib
 
 from .test_neural_gpu import _random_params, _synthetic_records
 
@@ -54,3 +57,24 @@ def test_training_step_is_adam_on_the_gradient(renderer):
     big = np.abs(g) > 0.3 * np.abs(g).max()  # far from zero: a resampled batch keeps their sign
     assert big.sum() > 5 and np.all(np.sign(step[big]) == -np.sign(g[big]))
     assert np.allclose(np.abs(step[big]), 1e-3, rtol=1e-2)
+
+
+def _free_memory():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert _lib.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0  # librhip's own HIP runtime
+    return free.value
+
+
+def test_large_calls_give_their_buffers_back(renderer):
+    """The outputs of 3M records (36 MB) are the call's own memory: after it, at most what a device may keep is gone."""
+    n = 3_000_000
+    print(f"[gpu] evaluation of {n} records", flush=True)
+    renderer.neural_records(n)
+    renderer.neural_write_records(0, np.tile(_synthetic_records(1000, 2), (n // 1000, 1)))
+    renderer.neural_set_weights(_random_params(6))
+    _, _, few = renderer.neural_evaluate(0, 1000, outputs=True)
+    before = _free_memory()
+    for _ in range(2):
+        _, _, out = renderer.neural_evaluate(0, n, outputs=True)
+        assert np.array_equal(out[:1000], few) and np.array_equal(out[-1000:], few)
+        assert before - _free_memory() <= 16 << 20
