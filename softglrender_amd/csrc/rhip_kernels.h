@@ -340,17 +340,9 @@ __device__ __forceinline__ int binClass(const DrawParams &P, int tx0, int ty0, i
   return kPrimGlobal;
 }
 
-/* Counts (EMIT false) or lists (EMIT true) primitive `id` in each of its bins. */
-template <bool EMIT>
-__device__ __forceinline__ void binVisit(const DrawParams &P, int id, int cls, int tx0, int ty0, int tx1, int ty1) {
-  auto put = [&](int b) {
-    if (EMIT) {
-      const int slot = atomicAdd(&P.bin_cursor[b], 1);
-      P.bin_items[P.bin_start[b] + slot] = id;
-    } else {
-      atomicAdd(&P.bin_count[b], 1);
-    }
-  };
+/* Counts a primitive in each of its bins. */
+__device__ __forceinline__ void binVisit(const DrawParams &P, int cls, int tx0, int ty0, int tx1, int ty1) {
+  auto put = [&](int b) { atomicAdd(&P.bin_count[b], 1); };
   if (cls == kPrimGlobal) {
     put(P.nbins - 1);
   } else if (cls == kPrimCoarse) {
@@ -435,13 +427,13 @@ __device__ __forceinline__ BinRect setupPrimAt(const DrawParams &P, int id, int 
     P.prims[id].flags = flags; /* nothing reads more of a primitive that is not live */
   return r;
 }
-__device__ BinRect setupPrim(const DrawParams &P, int id, int i0, int i1, int i2, int src = -1) {
-  return setupPrimAt(P, id, i0, i1, i2, P.frag[i0], P.frag[i1], P.frag[i2], src);
+__device__ BinRect setupPrim(const DrawParams &P, int id, int i0, int i1, int i2) {
+  return setupPrimAt(P, id, i0, i1, i2, P.frag[i0], P.frag[i1], P.frag[i2], -1);
 }
 
 /* Counts a primitive in its bins with plain atomics (for divergent callers). */
 __device__ __forceinline__ void binCount(const DrawParams &P, const BinRect &r) {
-  if (r.cls >= 0) binVisit<false>(P, 0, r.cls, r.tx0, r.ty0, r.tx1, r.ty1);
+  if (r.cls >= 0) binVisit(P, r.cls, r.tx0, r.ty0, r.tx1, r.ty1);
 }
 
 /* Bins of a primitive's BinRect: how many, and the k-th (row-major). */
@@ -2335,7 +2327,14 @@ __device__ __forceinline__ uint32_t pairQuads(const DrawParams &P, const Tri &T,
  * took 142 us each to list (now 88: a tile's chain of loads, bin to triangle to
  * vertex, at three workgroups per CU). Its tiles join the list of tiles with
  * fragments one atomic per workgroup. True if the tile has any. */
-constexpr int kListDirect = 8; /* a byte of quads and samples each in a lane's 64 bits */
+/* Entries up to which a tile is walked pixel by pixel: a lane's 64 bits hold a byte of quads and samples for each of
+ * eight. What the pixel walk costs depends on the entries, what the pairs cost on the pixels these cover. k_ord_list at
+ * 1366 x 768, pixel by pixel against in pairs, us: one or two clipped triangles that cover all (3 and 6 entries) 108 and
+ * 128 against 116 and 148, 4x 119 and 147 against 131 and 165; in every tile 1, 2, 4 and 8 triangles of some 8 pixels
+ * each 115, 113, 115 and 117 against 131, 113, 107 and 109, 4x 119, 123, 124 and 152 against 124, 107, 108 and 117. The
+ * line is drawn for the passes over the whole target, the most common draws here; both are below what the pairs took
+ * with one list atomic per tile (small triangles 195 to 209, 4x 190 to 198). */
+constexpr int kListDirect = 8;
 template <int S>
 __device__ __forceinline__ bool listTile(const DrawParams &P, int tile) {
   __shared__ uint32_t win[kOrdWin];
@@ -2366,8 +2365,6 @@ __device__ __forceinline__ bool listTile(const DrawParams &P, int tile) {
     if (lp == 0) P.ord_state[tile] = kOrdEmpty;
     return false;
   }
-  const float lx[4] = {0.375f, 0.875f, 0.125f, 0.625f};
-  const float ly[4] = {0.875f, 0.625f, 0.375f, 0.125f};
   float dep[S];
 #pragma unroll
   for (int s = 0; s < S; s++) {

@@ -25,10 +25,18 @@ namespace rhip {
 
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 
+/* Measured with reads of 64 KiB to 31.6 MiB, us:
+ *   pieces   256 KiB: 1 MiB 52, 8 MiB 307, 31.6 MiB 1,240; 512 KiB: 54, 242, 890; 1 MiB: 68, 234, 767; 2 MiB: 67, 252, 733
+ *   slots    8, 16 and 32 alike at every size; 16 are as many as a full HD image has pieces, twice
+ *   helpers  1: 8 MiB 271, 31.6 MiB 1,030; 2: 226, 764 to 814; 3: 234, 767; 5: 235, 769
+ *   line     with the helpers (from the first byte) 1 MiB 81, 2 MiB 100, 3 MiB 124, 4 MiB 145; without 67, 104, 143, 183 */
 constexpr size_t kSlotBytes = (size_t)1 << 20;
 constexpr int kSlots = 16;
-constexpr size_t kSmallBytes = (size_t)256 << 10; /* reads up to here take a ring of one slot of this size */
+constexpr int kHelpers = 3;
 constexpr size_t kParallelBytes = (size_t)2 << 20; /* larger reads are copied out by the helpers */
+/* Reads up to here take a ring of one slot of this size: a program that reads a few numbers or thumbnails pins 260 KiB and
+ * not 16 MiB (its first read takes about the same, 45 us; one that also reads larger images pays 35 us for the second ring). */
+constexpr size_t kSmallBytes = (size_t)256 << 10;
 constexpr int kRingErrors = 4;                     /* the device's error words come along with the first piece */
 constexpr int kNoPinned = 1;                       /* readPieces: pinned memory was refused, nothing was queued */
 
@@ -179,7 +187,7 @@ inline Copiers *copiers() {
   Shared &s = shared();
   std::lock_guard<std::mutex> l(s.m);
   if (!s.copiers) {
-    const int n = std::min(3, (int)std::thread::hardware_concurrency() / 2);
+    const int n = std::min(kHelpers, (int)std::thread::hardware_concurrency() / 2);
     std::unique_ptr<Copiers> c(new Copiers());
     try {
       for (int i = 0; i < n; i++) c->threads.emplace_back([q = c.get()] { q->run(); });
