@@ -320,7 +320,10 @@ static __global__ __launch_bounds__(256) void k_pl_sort(const int2 *where, const
  * r starts r moves on. Lane j takes the unit in place j, so that the lanes of a
  * wavefront have few vertices: all m units of one are compared with all m by
  * loads that the lanes share and that wait for nothing. A linked list per vertex,
- * walked by each of its units, needs no places but a chain of m loads a lane. */
+ * walked by each of its units, needs no places but a chain of m loads a lane; a
+ * sort of all points by vertex ten passes over them. A draw of a million points,
+ * every 64th on one vertex: 8.8 ms (list 18.3, sort 11.6, and 6.9 of each the
+ * one pixel's fragments); each on its own vertex 700 us (list 653, sort 845). */
 static __global__ __launch_bounds__(256) void k_pl_points(DrawParams P, PlUnit *units, const int *vcount, const int *vstart,
                                                          const int *sorted, unsigned long long *count, int has_colour) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;

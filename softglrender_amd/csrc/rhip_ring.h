@@ -13,9 +13,9 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -143,6 +143,7 @@ struct Shared {
   std::vector<std::unique_ptr<Ring>> free_rings;
   std::unique_ptr<Copiers> copiers;
   int devices = 0;
+  Shared() { free_rings.reserve(2 * kKeptRings); } /* giving a ring back allocates nothing */
 };
 /* never destroyed: a process may end with devices alive and helpers asleep */
 inline Shared &shared() {
@@ -182,18 +183,21 @@ struct RingLease {
   }
 };
 
-/* The helpers, started on first use (null where the host has no cores to spare or starts no thread). */
-inline Copiers *copiers() {
+/* The helpers, started on first use. Null where the host has no cores to spare, starts no thread or has no memory for
+ * them: a read that has queued its pieces goes on without them, so nothing may be thrown here. */
+inline Copiers *copiers() noexcept {
   Shared &s = shared();
   std::lock_guard<std::mutex> l(s.m);
   if (!s.copiers) {
     const int n = std::min(kHelpers, (int)std::thread::hardware_concurrency() / 2);
-    std::unique_ptr<Copiers> c(new Copiers());
+    std::unique_ptr<Copiers> c;
     try {
+      c.reset(new Copiers());
+      c->threads.reserve(n); /* before any thread is: one that runs must not be dropped */
       for (int i = 0; i < n; i++) c->threads.emplace_back([q = c.get()] { q->run(); });
-    } catch (const std::system_error &) {
+    } catch (const std::exception &) {
     }
-    if (c->threads.empty()) return nullptr;
+    if (!c || c->threads.empty()) return nullptr;
     s.copiers = std::move(c);
   }
   return s.copiers.get();

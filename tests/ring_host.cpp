@@ -4,6 +4,10 @@
  * complete in order, and allocations can be told to fail.
  * Usage: ring_host <check>; prints "ok" and returns 0, or says what differed.
  */
+#include <dlfcn.h>
+#include <errno.h>
+#include <pthread.h>
+
 #include <chrono>
 #include <cstdarg>
 #include <cstdio>
@@ -11,6 +15,7 @@
 #include <ctime>
 #include <deque>
 #include <functional>
+#include <new>
 #include <string>
 
 #include "rhip_ring.h"
@@ -118,6 +123,25 @@ hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, hipMemcpyKind, h
   return hipSuccess;
 }
 const char *hipGetErrorString(hipError_t) { return "error"; }
+}
+
+/* ------------------------------------------------------------------ refused memory and threads */
+
+namespace {
+thread_local int news_left = 1 << 30; /* allocations of this thread that still succeed */
+int threads_left = 1 << 30;           /* threads that can still be started */
+}  // namespace
+void *operator new(size_t n) {
+  if (news_left-- <= 0) throw std::bad_alloc();
+  if (void *p = malloc(n)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
+extern "C" int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(void *), void *arg) {
+  if (threads_left-- <= 0) return EAGAIN;
+  static auto real = (decltype(&pthread_create))dlsym(RTLD_NEXT, "pthread_create");
+  return real(t, a, f, arg);
 }
 
 namespace rhip {
@@ -293,6 +317,29 @@ int checkRefused() {
   return out[30] != 77 || memcmp(errors, dev_errors, sizeof errors);
 }
 
+/* Helpers that cannot be started, or not all, change no read and throw nothing. */
+int checkHelpers() {
+  if (read(64, 1)) return 1; /* the stream's own thread runs */
+  for (int k = 0; k < 6; k++) {
+    news_left = k;
+    Copiers *c = copiers();
+    news_left = 1 << 30;
+    if (k == 0 && c) return printf("helpers without memory\n"), 1;
+    if (read(20 * kSlotBytes, 10 + k)) return 1;
+    readDeviceGone();
+    readDeviceAdded();
+  }
+  for (int k = 0; k < kHelpers; k++) {
+    threads_left = k;
+    const int bad = read(20 * kSlotBytes + 4, 20 + k);
+    threads_left = 1 << 30;
+    if (bad) return 1;
+    readDeviceGone();
+    readDeviceAdded();
+  }
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -303,6 +350,7 @@ int main(int argc, char **argv) {
   if (what == "events") bad = checkEvents();
   if (what == "idle") bad = checkIdle();
   if (what == "refused") bad = checkRefused();
+  if (what == "helpers") bad = checkHelpers();
   readDeviceGone();
   if (!bad && pinned_blocks) {
     printf("%d pinned blocks left\n", pinned_blocks);
