@@ -549,14 +549,19 @@ __device__ __forceinline__ void setupBody(const DrawParams &P, int blk) {
     }
   }
   binBlock<false>(P, t, r);
+  /* room in the list with one atomic for the workgroup: they all go to one address */
+  __shared__ int s_need[4], s_at;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const unsigned long long nb = __ballot(needs);
-  if (nb) {
-    const int lane = threadIdx.x & 63, leader = __ffsll(nb) - 1;
-    int at = 0;
-    if (lane == leader) at = atomicAdd(&P.dcount[kCountClip], __popcll(nb));
-    at = __shfl(at, leader, 64);
-    if (needs) P.clip_list[at + __popcll(nb & ((1ull << lane) - 1ull))] = t;
-  }
+  if (lane == 0) s_need[wave] = __popcll(nb);
+  __syncthreads();
+  const int all = s_need[0] + s_need[1] + s_need[2] + s_need[3];
+  if (!all) return;
+  if (threadIdx.x == 0) s_at = atomicAdd(&P.dcount[kCountClip], all);
+  __syncthreads();
+  int at = s_at + __popcll(nb & ((1ull << lane) - 1ull));
+  for (int w = 0; w < wave; w++) at += s_need[w];
+  if (needs) P.clip_list[at] = t;
 }
 
 /* --------------------------------------------------------------------------- clipping */
@@ -729,7 +734,9 @@ __device__ void clipBody(const DrawParams &P, int blk, int nblocks) {
 }
 
 static __global__ __launch_bounds__(256) void k_setup(DrawParams P) { setupBody(P, xcdBlock(blockIdx.x, gridDim.x)); }
-static __global__ __launch_bounds__(256) void k_clip(DrawParams P) { clipBody(P, blockIdx.x, gridDim.x); }
+/* Five workgroups a CU (96 registers): a million clipped triangles 461 us with four, 418 with five, and 522 and 640 with six
+ * and eight, which spill. */
+static __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_clip(DrawParams P) { clipBody(P, blockIdx.x, gridDim.x); }
 
 /* --------------------------------------------------------------------------- binning */
 
@@ -745,26 +752,42 @@ __device__ __forceinline__ void binScanBody(const DrawParams &P) {
 
 static __global__ __launch_bounds__(1024) void k_bin_scan(DrawParams P) { binScanBody(P); }
 
-/* Lists every live primitive in its bins: the originals, then the clipped triangles' fans. */
+/* Lists primitive `id` (where `is`) in its bins; every thread of the workgroup calls it. */
+__device__ __forceinline__ void binEmitPrim(const DrawParams &P, int id, bool is) {
+  BinRect r = {-1, 0, 0, 0, 0};
+  if (is) {
+    const PrimSetup &ps = P.prims[id];
+    if (ps.flags & kPrimLive) {
+      tileRect(P, ps, r.tx0, r.ty0, r.tx1, r.ty1);
+      r.cls = ps.flags & (kPrimCoarse | kPrimGlobal);
+    }
+  }
+  binBlock<true>(P, id, r);
+}
+
+/* Lists every live primitive in its bins: the originals, then the clipped triangles' fans. A few clipped triangles
+ * share one pass with the originals, a thread for each place a fan can have; most places are empty, so many clipped
+ * triangles are walked by one thread each, as many passes as the workgroup's longest fan has triangles. */
 __device__ __forceinline__ void binEmitBody(const DrawParams &P, int blk, int nblocks) {
-  const int n = P.ntris + P.dcount[kCountClip] * kMaxFans;
-  for (int b0 = blk * blockDim.x; b0 < n; b0 += nblocks * blockDim.x) {
+  const int nclip = P.dcount[kCountClip], stride = nblocks * blockDim.x;
+  const bool places = nclip <= stride / kMaxFans;
+  const int n = P.ntris + (places ? nclip * kMaxFans : 0);
+  auto fansOf = [&](int t) { return P.clip_poly[(size_t)t * (kMaxPoly + 1) + kMaxPoly] - 3; };
+  for (int b0 = blk * blockDim.x; b0 < n; b0 += stride) {
     int id = b0 + threadIdx.x;
-    BinRect r = {-1, 0, 0, 0, 0};
     bool is = id < n;
     if (is && id >= P.ntris) {
       const int m = id - P.ntris, t = P.clip_list[m / kMaxFans], k = m % kMaxFans;
-      is = k < P.clip_poly[(size_t)t * (kMaxPoly + 1) + kMaxPoly] - 3;
+      is = k < fansOf(t);
       id = fanId(P, t, k);
     }
-    if (is) {
-      const PrimSetup &ps = P.prims[id];
-      if (ps.flags & kPrimLive) {
-        tileRect(P, ps, r.tx0, r.ty0, r.tx1, r.ty1);
-        r.cls = ps.flags & (kPrimCoarse | kPrimGlobal);
-      }
-    }
-    binBlock<true>(P, id, r);
+    binEmitPrim(P, id, is);
+  }
+  if (places) return;
+  for (int b0 = blk * blockDim.x; b0 < nclip; b0 += stride) {
+    const int m = b0 + threadIdx.x, t = m < nclip ? P.clip_list[m] : 0;
+    const int fans = m < nclip ? fansOf(t) : 0;
+    for (int k = 0; __syncthreads_or(k < fans); k++) binEmitPrim(P, fanId(P, t, k), k < fans);
   }
 }
 
