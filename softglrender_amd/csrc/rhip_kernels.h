@@ -485,15 +485,17 @@ __device__ __forceinline__ int binSlot(BinHash &H, int b, bool insert) {
  * with one global atomic per distinct bin of the workgroup: pairs are counted
  * per bin in LDS, each bin reserves its range once, and the pairs fill it. A
  * bin the table cannot hold takes a global atomic per pair. Every thread of
- * the workgroup must call it (r.cls < 0: no bins). */
-template <bool EMIT>
-__device__ void binBlock(const DrawParams &P, int id, const BinRect &r) {
+ * the workgroup must call it (r.cls < 0: no bins). `first` is called after the
+ * first of its barriers: what it writes to LDS all threads see afterwards. */
+template <bool EMIT, typename First>
+__device__ __forceinline__ void binBlock(const DrawParams &P, int id, const BinRect &r, First first) {
   __shared__ BinHash H;
   for (int i = threadIdx.x; i < kBinHash; i += blockDim.x) {
     H.bin[i] = -1;
     H.cnt[i] = 0;
   }
   __syncthreads();
+  first();
   const int nb = binsOf(P, r);
   for (int k = 0; k < nb; k++) {
     const int b = binAt(P, r, k);
@@ -548,17 +550,18 @@ __device__ __forceinline__ void setupBody(const DrawParams &P, int blk) {
       r = setupPrim(P, t, i0, i1, i2);
     }
   }
-  binBlock<false>(P, t, r);
-  /* room in the list with one atomic for the workgroup: they all go to one address */
+  /* room in the clip list with one atomic for the workgroup, as they all go to one address; its latency and the counts'
+   * exchange run behind the binning's own barriers */
   __shared__ int s_need[4], s_at;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const unsigned long long nb = __ballot(needs);
   if (lane == 0) s_need[wave] = __popcll(nb);
-  __syncthreads();
-  const int all = s_need[0] + s_need[1] + s_need[2] + s_need[3];
-  if (!all) return;
-  if (threadIdx.x == 0) s_at = atomicAdd(&P.dcount[kCountClip], all);
-  __syncthreads();
+  binBlock<false>(P, t, r, [&] {
+    if (threadIdx.x) return;
+    const int all = s_need[0] + s_need[1] + s_need[2] + s_need[3];
+    if (all) s_at = atomicAdd(&P.dcount[kCountClip], all);
+  });
+  if (!nb) return;
   int at = s_at + __popcll(nb & ((1ull << lane) - 1ull));
   for (int w = 0; w < wave; w++) at += s_need[w];
   if (needs) P.clip_list[at] = t;
@@ -608,10 +611,11 @@ __device__ __forceinline__ void binCountWave(const DrawParams &P, const BinRect 
  * up triangle q of the fan. Triangle t's new vertices take slots nverts + t *
  * kMaxClipVerts onward. Latency bounds it: with one thread per triangle, whose
  * polygon lay in scratch memory, in the setup kernel, that kernel took 52 us for
- * the twelve triangles of a skybox or an IBL map's pass (now 5.5 us, and 13.8 us
+ * the twelve triangles of a skybox or an IBL map's pass (now 5.6 us, and 13.9 us
  * here), then the fans another launch after a scan; for 2M random triangles with
- * 5,490 to clip 195 us (161 us and 19 us, the lighter setup fits 8 wavefronts a
- * SIMD instead of 5). */
+ * 5,490 to clip 195 us (154 us and 19 us, the lighter setup fits 8 wavefronts a
+ * SIMD instead of 5). Where all of a million triangles clip it took 417 us and
+ * the fans 57; now 61 us and 418 us. */
 __device__ void clipBody(const DrawParams &P, int blk, int nblocks) {
   __shared__ ClipLds L;
   const int n = P.dcount[kCountClip];
@@ -762,7 +766,7 @@ __device__ __forceinline__ void binEmitPrim(const DrawParams &P, int id, bool is
       r.cls = ps.flags & (kPrimCoarse | kPrimGlobal);
     }
   }
-  binBlock<true>(P, id, r);
+  binBlock<true>(P, id, r, [] {});
 }
 
 /* Lists every live primitive in its bins: the originals, then the clipped triangles' fans. A few clipped triangles
