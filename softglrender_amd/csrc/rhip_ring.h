@@ -232,14 +232,15 @@ int readPieces(int hip_device, hipStream_t stream, size_t bytes, void *out, uint
   while (issued < std::min(pieces, kSlots) && he == hipSuccess) issue();
   if (he != hipSuccess) return give_up();
 
-  /* the work queued before the read is waited for here, and only then are helpers woken: they never spin through it */
+  /* the work queued before the read is waited for here, with the first piece, and only then are helpers woken: they never
+   * spin through it */
   if ((he = hipEventSynchronize(R.ev[0])) != hipSuccess) return give_up();
   Copiers *C = bytes > kParallelBytes ? copiers() : nullptr;
   std::unique_lock<std::mutex> own;
   if (C) own = std::unique_lock<std::mutex>(C->owner, std::try_to_lock);
   if (!C || !own.owns_lock()) {
     for (int c = 0; c < pieces; c++) {
-      if ((he = hipEventSynchronize(R.ev[c % kSlots])) != hipSuccess) return give_up();
+      if (c && (he = hipEventSynchronize(R.ev[c % kSlots])) != hipSuccess) return give_up();
       const size_t at = (size_t)c * kSlotBytes;
       memcpy((char *)out + at, R.slots + (size_t)(c % kSlots) * kSlotBytes, std::min(kSlotBytes, bytes - at));
       if (issued < pieces) {
@@ -250,7 +251,7 @@ int readPieces(int hip_device, hipStream_t stream, size_t bytes, void *out, uint
   } else {
     C->start(R.slots, out, bytes, pieces);
     for (int c = 0; c < pieces && he == hipSuccess; c++) {
-      he = hipEventSynchronize(R.ev[c % kSlots]);
+      if (c) he = hipEventSynchronize(R.ev[c % kSlots]);
       if (he != hipSuccess) break;
       C->ready.store(c + 1, std::memory_order_release);
       /* half a ring ahead of the copies: piece p + kSlots goes into p's slot once p is out of it */
